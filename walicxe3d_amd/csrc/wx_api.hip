@@ -103,8 +103,11 @@ struct Ctx {
   // device memory
   BlockInfo *d_info = nullptr;
   double *d_tabT = nullptr, *d_tabC = nullptr;
-  double *dU = nullptr, *dUP = nullptr, *dP = nullptr, *dF = nullptr, *dTmp = nullptr;
+  // plain form; dP and dP2 swap when a second stage's primitives replace the first's
+  double *dU = nullptr, *dUP = nullptr, *dP = nullptr, *dP2 = nullptr;
   unsigned long long *d_scal = nullptr;  // [0] dt bits, [1] floor count
+  unsigned long long *d_slots = nullptr; // plain form: partial minima of dt (DT_SLOTS)
+  StepState *d_ss = nullptr;             // plain form: the step's scalars
   bool have_state = false;
   bool ghosts_recorded = false;      // fused form: ghost layer of wx_record_ghosts in d_ghosts
   double *d_ghosts = nullptr;        // [blk][rho, p][6][256]
@@ -124,10 +127,9 @@ void free_mesh(Ctx *c) {
   hipFree(c->dU);
   hipFree(c->dUP);
   hipFree(c->dP);
-  hipFree(c->dF);
-  hipFree(c->dTmp);
+  hipFree(c->dP2);
   c->d_info = nullptr;
-  c->dU = c->dUP = c->dP = c->dF = c->dTmp = nullptr;
+  c->dU = c->dUP = c->dP = c->dP2 = nullptr;
   fused_free(c->fused);
   hipFree(c->d_ghosts);
   hipFree(c->d_mark);
@@ -307,18 +309,27 @@ void fill_devcfg(Ctx *c, const double *dxyz) {
 }
 
 __global__ void k_scatter(int nv, int nblk, const double *src, double *dst, int zero_ghosts) {
-  // one thread per stored cell: dst [blk][nv][20^3] <- src [blk][nv][16^3]
+  // one thread per stored cell: dst [blk][nv][NSTORE] <- src [blk][nv][16^3]
   size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  size_t total = (size_t)nblk * nv * NCELL;
+  size_t total = (size_t)nblk * nv * NSTORE;
   if (t >= total) return;
-  int q = (int)(t % NCELL);
-  size_t bv = t / NCELL;
-  int i = q % NB - 1, j = (q / NB) % NB - 1, k = q / (NB * NB) - 1;
-  bool in = i >= 1 && i <= NC && j >= 1 && j <= NC && k >= 1 && k <= NC;
-  if (in)
-    dst[t] = src[bv * NINT + ((k - 1) * NC + (j - 1)) * NC + (i - 1)];
+  int q = (int)(t % NSTORE);
+  size_t bv = t / NSTORE;
+  if (q < NINT)
+    dst[t] = src[bv * NINT + q];
   else if (zero_ghosts)
     dst[t] = 0.0;
+}
+
+// the arrays with ghosts as 20^3 cubes (edge and corner ghosts, which nothing
+// fills or reads, are zero)
+__global__ void k_cubes(size_t cubes, const double *src, double *dst) {
+  size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= cubes * NCELL) return;
+  const int q = (int)(t % NCELL);
+  const int i = q % NB - 1, j = (q / NB) % NB - 1, k = q / (NB * NB) - 1;
+  const int outside = (i < 1 || i > NC) + (j < 1 || j > NC) + (k < 1 || k > NC);
+  dst[t] = outside > 1 ? 0.0 : src[(t / NCELL) * NSTORE + cid(i, j, k)];
 }
 
 __global__ void k_gather(int nv, int nblk, const double *src, double *dst) {
@@ -327,8 +338,7 @@ __global__ void k_gather(int nv, int nblk, const double *src, double *dst) {
   if (t >= total) return;
   int q = (int)(t % NINT);
   size_t bv = t / NINT;
-  int i = q % NC + 1, j = (q / NC) % NC + 1, k = q / (NC * NC) + 1;
-  dst[t] = src[bv * NCELL + cid(i, j, k)];
+  dst[t] = src[bv * NSTORE + q];
 }
 
 int launch_check(const char *what);
@@ -474,8 +484,7 @@ int launch_check(const char *what) {
 
 // ------------------------- plain-form sequences ----------------------------
 int plain_timestep_raw(Ctx *c, double *dt) {
-  HIPCHK(hipMemsetAsync(c->d_scal, 0xFF, sizeof(unsigned long long), c->st));
-  plain_timestep(c->dc, c->dP, c->d_scal, c->st);
+  plain_timestep(c->dc, c->dP, c->d_slots, c->d_scal, c->st);
   unsigned long long bits = 0;
   HIPCHK(hipMemcpyAsync(&bits, c->d_scal, sizeof(bits), hipMemcpyDeviceToHost, c->st));
   HIPCHK(hipStreamSynchronize(c->st));
@@ -490,19 +499,51 @@ int plain_timestep_raw(Ctx *c, double *dt) {
   return WX_OK;
 }
 
-int plain_godunov(Ctx *c, int order, double dt) {
-  double dtp = order == 2 ? dt / 2.0 : dt;
-  plain_boundary(c->dc, plane_wind(c), c->dU, 1, c->st);
-  plain_prims(c->dc, c->dU, c->dP, WX_CELLS_GHOST, nullptr, c->st);
-  plain_fluxes(c->dc, c->dP, c->dF, 1, c->st);
-  plain_upwind(c->dc, c->us, c->dU, c->dP, c->dF, c->dUP, dtp, c->st);
+// Godunov(order) over dt, or over the device's dt with ss.  The second
+// stage's primitives go to the other PRIM array: the first stage's update
+// writes them while its neighbours still read theirs.
+void plain_stages(Ctx *c, int order, const StepState *ss, double dt) {
+  const PlaneWind pw = plane_wind(c);
+  plain_ghosts(c->dc, pw, c->dU, c->dP, c->dP, 1, nullptr, c->st);
+  plain_update(c->dc, c->us, c->dU, c->dP, c->dUP, order == 2 ? c->dP2 : nullptr, ss, dt, order == 2, 1, c->st);
   if (order == 2) {
-    plain_boundary(c->dc, plane_wind(c), c->dUP, 2, c->st);
-    plain_prims(c->dc, c->dUP, c->dP, WX_CELLS_ALL, nullptr, c->st);
-    plain_fluxes(c->dc, c->dP, c->dF, 2, c->st);
-    plain_upwind(c->dc, c->us, c->dU, c->dP, c->dF, c->dUP, dt, c->st);
+    plain_ghosts(c->dc, pw, c->dUP, c->dP2, c->dP, 2, c->dP2, c->st);
+    plain_update(c->dc, c->us, c->dU, c->dP2, c->dUP, nullptr, ss, dt, 0, 2, c->st);
+    std::swap(c->dP, c->dP2);
   }
+}
+
+int plain_godunov(Ctx *c, int order, double dt) {
+  plain_stages(c, order, nullptr, dt);
   return launch_check("godunov");
+}
+
+// nsteps iterations of the main loop with the scalars on the device: one
+// transfer in, one out, no synchronisation between steps (two per step
+// before, for dt and the floor count).  Returns the last step's floor count.
+int plain_steps(Ctx *c, int nsteps, int *it, double *dt, double *time, int *nextout, double dtout, double t_sc) {
+  StepState s{};
+  s.it = *it;
+  s.time = *time;
+  s.nextout = *nextout;
+  s.dtout = dtout;
+  s.t_sc = t_sc;
+  HIPCHK(hipMemcpyAsync(c->d_ss, &s, sizeof(s), hipMemcpyHostToDevice, c->st));
+  for (int n = 0; n < nsteps; n++) {
+    plain_step_begin(c->dc, n == 0 ? c->dP : nullptr, c->d_ss, c->d_slots, n > 0, c->st);
+    plain_stages(c, c->cfg.solver == SOLVER_HLL1 ? 1 : 2, c->d_ss, 0.0);
+    plain_finish(c->dc, c->dUP, c->dU, c->dP, c->d_ss, c->cfg.mu0, n + 1 < nsteps ? c->d_slots : nullptr, c->st);
+  }
+  int rc = launch_check("step");
+  if (rc != WX_OK) return rc;
+  HIPCHK(hipMemcpyAsync(&s, c->d_ss, sizeof(s), hipMemcpyDeviceToHost, c->st));
+  HIPCHK(hipStreamSynchronize(c->st));
+  step_close(&s);
+  *it = s.it;
+  *dt = s.dt;
+  *time = s.time;
+  *nextout = s.nextout;
+  return (int)s.floors;
 }
 
 int update_prims(Ctx *c, long *bad) {
@@ -636,7 +677,7 @@ __global__ void __launch_bounds__(256) k_carry_prims(int nv, const RemapSrc *map
   if (map[b].kind == 2) return;
   const int i = threadIdx.x & 15, j = threadIdx.x >> 4;
   const double *S = src + ((size_t)b * nv + v) * NINT;
-  double *D = P + ((size_t)b * nv + v) * NCELL;
+  double *D = P + ((size_t)b * nv + v) * NSTORE;
   for (int k = 0; k < NC; k++) D[cid(i + 1, j + 1, k + 1)] = S[(k * NC + j) * NC + i];
 }
 
@@ -882,7 +923,13 @@ int wx_init(const wx_config *cfg, void **out) {
     delete c;
     return fail(WX_EHIP, "stream creation failed");
   }
-  if (hipMalloc(&c->d_scal, 4 * sizeof(unsigned long long)) != hipSuccess) {
+  const size_t slot_bytes = DT_SLOTS * DT_STRIDE * sizeof(unsigned long long);
+  if (hipMalloc(&c->d_scal, 4 * sizeof(unsigned long long)) != hipSuccess ||
+      hipMalloc(&c->d_slots, slot_bytes) != hipSuccess || hipMalloc(&c->d_ss, sizeof(StepState)) != hipSuccess ||
+      hipMemsetAsync(c->d_slots, 0xFF, slot_bytes, c->st) != hipSuccess) {
+    hipFree(c->d_scal);
+    hipFree(c->d_slots);
+    hipFree(c->d_ss);
     hipStreamDestroy(c->st);
     delete c;
     return fail(WX_ENOMEM, "device allocation failed");
@@ -904,6 +951,8 @@ int wx_finalize(void *ctx) {
   hipStreamSynchronize(c->st);
   free_mesh(c);
   hipFree(c->d_scal);
+  hipFree(c->d_slots);
+  hipFree(c->d_ss);
   hipFree(c->d_tabT);
   hipFree(c->d_tabC);
   hipFree(c->d_stage);
@@ -934,7 +983,7 @@ static int set_mesh_impl(Ctx *c, const int nroot[3], int maxlev, const double *d
     rc = build_topology(c, bids);
   }
   if (rc != WX_OK) return rc;
-  size_t n = (size_t)nblk * c->cfg.nv * NCELL;
+  size_t n = (size_t)nblk * c->cfg.nv * NSTORE;
   HIPCHK(hipMalloc(&c->d_info, sizeof(BlockInfo) * nblk));
   HIPCHK(hipMemcpy(c->d_info, c->info.data(), sizeof(BlockInfo) * nblk, hipMemcpyHostToDevice));
   if (!is_fused(c)) {
@@ -945,7 +994,8 @@ static int set_mesh_impl(Ctx *c, const int nroot[3], int maxlev, const double *d
     HIPCHK(hipMemset(c->dP, 0, n * sizeof(double)));
     HIPCHK(hipMalloc(&c->dUP, n * sizeof(double)));
     HIPCHK(hipMemset(c->dUP, 0, n * sizeof(double)));
-    HIPCHK(hipMalloc(&c->dF, plain_flux_elems(nblk, c->cfg.nv) * sizeof(double)));
+    HIPCHK(hipMalloc(&c->dP2, n * sizeof(double)));
+    HIPCHK(hipMemsetAsync(c->dP2, 0, n * sizeof(double), c->st));
   }
   fill_devcfg(c, dxyz);
   if (is_fused(c)) {
@@ -976,7 +1026,7 @@ static int upload_device(Ctx *c, double *d_in, bool adopt = false) {
     c->have_state = true;
     return WX_OK;
   }
-  size_t total = (size_t)c->nblk * nv * NCELL;
+  size_t total = (size_t)c->nblk * nv * NSTORE;
   hipLaunchKernelGGL(k_scatter, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, c->st, nv, c->nblk, d_in, c->dU, 1);
   int rc = launch_check("upload");
   HIPCHK(hipStreamSynchronize(c->st));
@@ -1032,7 +1082,7 @@ int wx_upload_prims(void *ctx, const double *p, int layout, int nbmax, const int
   } else {
     HIPCHK(hipMemcpyAsync(d_in.p, p, ni * sizeof(double), hipMemcpyHostToDevice, c->st));
   }
-  size_t total = (size_t)c->nblk * nv * NCELL;
+  size_t total = (size_t)c->nblk * nv * NSTORE;
   const double *in = d_in.p;
   hipLaunchKernelGGL(k_scatter, dim3((unsigned)((total + 255) / 256)), dim3(256), 0, c->st, nv, c->nblk, in, c->dP, 0);
   rc = launch_check("upload_prims");
@@ -1134,30 +1184,7 @@ int wx_step(void *ctx, int *it, double *dt, double *time, int *nextout, double d
   if (rc != WX_OK) return rc;
   if (!it || !dt || !time || !nextout) return fail(WX_EINVAL, "null argument");
   if (is_fused(c)) return wx_run(ctx, 1, it, dt, time, nextout, dtout, t_sc);
-  *it += 1;
-  double dtl;
-  rc = plain_timestep_raw(c, &dtl);
-  if (rc != WX_OK) return rc;
-  // start-up ramp and output clamp (source/hydro_solver.f90:191-207)
-  if (*it <= 10) dtl = std::ldexp(1.0, -(11 - *it)) * dtl;
-  double tout = (double)(*nextout) * dtout / t_sc;
-  bool dump = false;
-  if (*time + dtl >= tout) {
-    dtl = tout - *time;
-    dump = true;
-  }
-  *dt = dtl;
-  rc = plain_godunov(c, c->cfg.solver == SOLVER_HLL1 ? 1 : 2, dtl);
-  if (rc != WX_OK) return rc;
-  *time = *time + dtl;
-  plain_viscous(c->dc, c->dUP, c->dU, c->st);
-  long bad = 0;
-  rc = update_prims(c, &bad);
-  if (rc != WX_OK) return rc;
-  if (c->cfg.cooling) plain_cooling(c->dc, c->dU, c->dP, dtl, c->cfg.mu0, c->st);
-  if (dump) *nextout += 1;
-  rc = launch_check("step");
-  return rc != WX_OK ? rc : (int)bad;
+  return plain_steps(c, 1, it, dt, time, nextout, dtout, t_sc);
 }
 
 int wx_run(void *ctx, int nsteps, int *it, double *dt, double *time, int *nextout, double dtout, double t_sc) {
@@ -1166,11 +1193,9 @@ int wx_run(void *ctx, int nsteps, int *it, double *dt, double *time, int *nextou
   if (rc != WX_OK) return rc;
   if (!it || !dt || !time || !nextout || nsteps < 0) return fail(WX_EINVAL, "bad argument");
   if (!is_fused(c)) {
-    for (int s = 0; s < nsteps; s++) {
-      rc = wx_step(ctx, it, dt, time, nextout, dtout, t_sc);
-      if (rc < 0) return rc;
-    }
-    return WX_OK;
+    if (nsteps == 0) return WX_OK;
+    rc = plain_steps(c, nsteps, it, dt, time, nextout, dtout, t_sc);
+    return rc < 0 ? rc : WX_OK;
   }
   int frc = fused_run(c->fused, c->dc, c->st, nsteps, it, dt, time, nextout, dtout, t_sc);
   if (frc) return fail(WX_EHIP, std::string("fused run failed: ") + fused_error());
@@ -1202,8 +1227,7 @@ int wx_fluxes_update(void *ctx, int order, double dtp) {
   int rc = need_state(c);
   if (rc != WX_OK) return rc;
   if (is_fused(c)) return fail(WX_EINVAL, "plain-form entry point");
-  plain_fluxes(c->dc, c->dP, c->dF, order, c->st);
-  plain_upwind(c->dc, c->us, c->dU, c->dP, c->dF, c->dUP, dtp, c->st);
+  plain_update(c->dc, c->us, c->dU, c->dP, c->dUP, nullptr, nullptr, dtp, 0, order == 2 ? 2 : 1, c->st);
   return launch_check("fluxes_update");
 }
 
@@ -1213,10 +1237,14 @@ int wx_copy_raw(void *ctx, int which, double *out) {
   if (rc != WX_OK) return rc;
   if (is_fused(c)) return fail(WX_EINVAL, "plain-form entry point");
   const double *src = which == 0 ? c->dU : which == 1 ? c->dUP : c->dP;
-  size_t n = (size_t)c->nblk * c->cfg.nv * NCELL;
-  HIPCHK(hipMemcpyAsync(out, src, n * sizeof(double), hipMemcpyDeviceToHost, c->st));
+  const size_t cubes = (size_t)c->nblk * c->cfg.nv, n = cubes * NCELL;
+  DevBuf<double> d_out;
+  HIPCHK(d_out.alloc(n));
+  double *to = d_out.p;
+  hipLaunchKernelGGL(k_cubes, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->st, cubes, src, to);
+  HIPCHK(hipMemcpyAsync(out, to, n * sizeof(double), hipMemcpyDeviceToHost, c->st));
   HIPCHK(hipStreamSynchronize(c->st));
-  return WX_OK;
+  return launch_check("copy_raw");
 }
 
 int wx_set_tuning(void *ctx, int kind, int value) {

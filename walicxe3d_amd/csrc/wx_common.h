@@ -10,6 +10,12 @@ constexpr int NG = 2;              // ghost layers (nghost)
 constexpr int NB = NC + 2 * NG;    // 20: stored edge with ghosts
 constexpr int NCELL = NB * NB * NB;
 constexpr int NINT = NC * NC * NC; // 4096 interior cells
+// The plain form stores a block's variable as its interior (i fastest), then
+// its face ghosts as 12 planes of 16 x 16: rows of the interior and of a
+// ghost plane fill whole 128-byte lines.  (In a 20^3 cube every row straddles
+// two lines and a ghost of an x face is alone in its line: the writes of
+// partial lines, shared between the chiplets' L2s, took most of the time.)
+constexpr int NSTORE = NINT + 12 * NC * NC;
 constexpr int MAXV = 8;
 
 // source/constants.f90:52-104
@@ -28,10 +34,18 @@ void wx_emu_check_failed(const char *what, const char *file, int line);
 #define WX_EMU_CHECK(c) ((void)0)
 #endif
 
-// Index of cell (i,j,k), i,j,k in [-1, 18] (reference bounds nxmin..nxmax)
+// Index of cell (i,j,k) in the plain form's arrays: the interior, or a face
+// ghost (one coordinate in [-1, 0] or [17, 18]; reference bounds
+// nxmin..nxmax).  Ghost planes: face x 2 + layer - 1, then the two transverse
+// coordinates, the lower axis fastest.
 __host__ __device__ constexpr inline int cid(int i, int j, int k) {
+  const bool xg = i < 1 || i > NC, yg = j < 1 || j > NC, zg = k < 1 || k > NC;
   WX_EMU_CHECK(i >= -1 && i <= NC + 2 && j >= -1 && j <= NC + 2 && k >= -1 && k <= NC + 2);
-  return ((k + 1) * NB + (j + 1)) * NB + (i + 1);
+  WX_EMU_CHECK((int)xg + (int)yg + (int)zg <= 1);
+  const int gx = i < 1 ? -i : i - NC + 1, gy = 4 + (j < 1 ? -j : j - NC + 1), gz = 8 + (k < 1 ? -k : k - NC + 1);
+  const int plane = xg ? gx : (yg ? gy : gz);
+  const int row = zg ? j - 1 : k - 1, col = xg ? j - 1 : i - 1;
+  return (xg || yg || zg) ? NINT + (plane * NC + row) * NC + col : ((k - 1) * NC + (j - 1)) * NC + (i - 1);
 }
 
 // One face of one block in the neighbour table.  For NEIGH_FINER the four

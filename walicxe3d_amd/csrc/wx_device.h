@@ -33,6 +33,46 @@ struct DevCfg {
   double winds[MAXWIND][8];
 };
 
+// Device-resident step scalars (the host never reads them between steps).
+struct StepState {
+  double dt;          // dt of the current step
+  double time;        // simulation time at the start of the step
+  double dtout;       // output interval (parameters dtout)
+  double t_sc;        // time unit (parameters t_sc)
+  unsigned long long dtmin_bits;  // running min of dx/(|v|+c) over cells (fused form)
+  int it;             // iteration counter
+  int nextout;        // next output number
+  int dump;           // the clamp fired this step
+  int pad;
+  unsigned long long floors;      // cells floored in the current step (plain form)
+};
+
+// words over which workgroups spread the smallest dt of the plain form (one
+// per 64-byte line)
+constexpr int DT_SLOTS = 64, DT_STRIDE = 8;
+
+// dt of a step from the smallest dx/(|v|+c): CFL, start-up ramp, output
+// clamp (source/hydro_solver.f90:183-207)
+__device__ inline void step_open(StepState *s, double m, double cfl, int cooling) {
+  double dtl = cooling ? fmin(m, 1.0e30) * cfl : m * cfl;
+  int it = s->it + 1;
+  s->it = it;
+  if (it <= 10) dtl = ldexp(1.0, -(11 - it)) * dtl;
+  double tout = (double)s->nextout * s->dtout / s->t_sc;
+  s->dump = 0;
+  if (s->time + dtl >= tout) {
+    dtl = tout - s->time;
+    s->dump = 1;
+  }
+  s->dt = dtl;
+  s->floors = 0;
+}
+
+__host__ __device__ inline void step_close(StepState *s) {
+  s->time = s->time + s->dt;
+  if (s->dump) s->nextout += 1;
+}
+
 // ---------------------------------------------------------------------------
 // Face exchange: where the value of a face ghost cell comes from.
 // Ghost layer g (1 adjacent, 2 outer) of face f of block b at transverse
@@ -119,10 +159,10 @@ __host__ __device__ inline bool ghost_source(const BlockInfo *info, const int *b
 }
 
 // Value of variable v of a face ghost from its source, reading an array
-// with ghosts ([blk][nv][20^3]) of element type T, computing in R.
+// with ghosts ([blk][nv][NSTORE]) of element type T, computing in R.
 template <typename R, typename T>
 __device__ inline R ghost_value(const T *A, int nv, const GhostSrc &s, int v) {
-  const T *S = A + ((size_t)s.blk * nv + v) * NCELL;
+  const T *S = A + ((size_t)s.blk * nv + v) * NSTORE;
   if (s.kind == 1) {
     R acc = R(0);
     for (int dx = 0; dx < 2; dx++)

@@ -11,19 +11,6 @@
 
 namespace wx {
 
-// Device-resident step scalars (the host never reads them between steps).
-struct StepState {
-  double dt;          // dt of the current step
-  double time;        // simulation time at the start of the step
-  double dtout;       // output interval (parameters dtout)
-  double t_sc;        // time unit (parameters t_sc)
-  unsigned long long dtmin_bits;  // running min of dx/(|v|+c) over cells
-  int it;             // iteration counter
-  int nextout;        // next output number
-  int dump;           // the clamp fired this step
-  int pad;
-};
-
 struct FusedState {
   double *U = nullptr;       // [blk][nv][4096] FP64 conserved state (the current one)
   // FP32 MHD form: UP holds FP32 increments over U^n, so the second stage

@@ -53,25 +53,11 @@ __global__ void __launch_bounds__(256) k_dt_init(FusedArgs a) {
 // dt of the step: CFL, start-up ramp, output clamp
 // (source/hydro_solver.f90:183-207); resets the running minimum
 __global__ void k_dt_finalize(StepState *s, double cfl, int cooling) {
-  double m = __longlong_as_double((long long)s->dtmin_bits);
-  double dtl = cooling ? fmin(m, 1.0e30) * cfl : m * cfl;
-  int it = s->it + 1;
-  s->it = it;
-  if (it <= 10) dtl = ldexp(1.0, -(11 - it)) * dtl;
-  double tout = (double)s->nextout * s->dtout / s->t_sc;
-  s->dump = 0;
-  if (s->time + dtl >= tout) {
-    dtl = tout - s->time;
-    s->dump = 1;
-  }
-  s->dt = dtl;
+  step_open(s, __longlong_as_double((long long)s->dtmin_bits), cfl, cooling);
   s->dtmin_bits = ~0ull;
 }
 
-__global__ void k_step_post(StepState *s) {
-  s->time = s->time + s->dt;
-  if (s->dump) s->nextout += 1;
-}
+__global__ void k_step_post(StepState *s) { step_close(s); }
 
 // PRIM of the state in the same layout ([blk][nv][16^3]), for downloads
 template <int NV>

@@ -215,6 +215,27 @@ __host__ __device__ inline void limit1_minmod32(float pll, float &pl, float &pr,
   pr = pr - 0.5f * ar;
 }
 
+// limit1 of NV variables, the option tested once instead of per variable
+template <int NV, typename R>
+__host__ __device__ inline void limit_all(const R *pll, R *pl, R *pr, const R *prr, int lim) {
+#define WX_LIMIT_CASE(L) \
+  case L:                \
+    for (int q = 0; q < NV; q++) limit1(pll[q], pl[q], pr[q], prr[q], L); \
+    break;
+  switch (lim) {
+    WX_LIMIT_CASE(-1)
+    WX_LIMIT_CASE(0)
+    WX_LIMIT_CASE(1)
+    WX_LIMIT_CASE(2)
+    WX_LIMIT_CASE(3)
+    WX_LIMIT_CASE(4)
+    WX_LIMIT_CASE(5)
+    default:
+    WX_LIMIT_CASE(6)
+  }
+#undef WX_LIMIT_CASE
+}
+
 // HLL / HLLE flux (source/hll.f90:175-215, source/hlle.f90:166-206);
 // strict selects the HLLE comparisons (sl > 0, sr < 0)
 template <typename R>
@@ -281,6 +302,45 @@ __host__ __device__ inline void primfhllc(const Phys<R> &c, const R *pL, const R
   ust[4] = rhost * (EK / pK[0] + (sst - pK[1]) * (sst + pK[4] / (pK[0] * (sK - pK[1]))));
   for (int q = 5; q < c.nv; q++) ust[q] = R(0);
   for (int q = 0; q < c.nv; q++) ff[q] = fK[q] + sK * (ust[q] - uK[q]);
+}
+
+// primfhllc with one code path for its four outcomes (the physical flux of
+// either side, or its star flux): the side K is picked with selects, its flux
+// is formed once.  Every value is the expression primfhllc uses, so the two
+// agree bit for bit; lanes of a wavefront on different sides of the contact no
+// longer run each side's code in turn, and no array is read through a pointer.
+template <typename R>
+__host__ __device__ inline void primfhllc_sel(const Phys<R> &c, const R *pL, const R *pR, R *ff) {
+  R dl1 = pL[0], dr1 = pR[0], ul1 = pL[1], ur1 = pR[1], pl1 = pL[4], pr1 = pR[4];
+  R cl = sound(c, pL), cr = sound(c, pR);
+  R sl = rfmin(ul1 - cl, ur1 - cr);
+  R sr = rfmax(ul1 + cl, ur1 + cr);
+  R sst = R(0);
+  if (c.solver == SOLVER_HLLC)
+    sst = (pr1 - pl1 + dl1 * ul1 * (sl - ul1) - dr1 * ur1 * (sr - ur1)) / (dl1 * (sl - ul1) - dr1 * (sr - ur1));
+  const bool supL = sl > R(0), supR = !supL && sr < R(0);
+  const bool isL = supL || (!supR && sst >= R(0));
+  R pK[MAXV], fK[MAXV], uK[MAXV];
+  for (int q = 0; q < c.nv; q++) pK[q] = isL ? pL[q] : pR[q];
+  const R sK = isL ? sl : sr;
+  xflux(c, pK, fK);
+  if (supL || supR) {
+    for (int q = 0; q < c.nv; q++) ff[q] = fK[q];
+    return;
+  }
+  prim2flow(c, pK, uK);
+  R ust[MAXV];
+  R rhost = pK[0] * (sK - pK[1]) / (sK - sst);
+  R EK = R(0.5) * pK[0] * (pK[1] * pK[1] + pK[2] * pK[2] + pK[3] * pK[3]) + c.cv * pK[4];
+  ust[0] = rhost;
+  ust[1] = rhost * sst;
+  ust[2] = rhost * pK[2];
+  ust[3] = rhost * pK[3];
+  ust[4] = rhost * (EK / pK[0] + (sst - pK[1]) * (sst + pK[4] / (pK[0] * (sK - pK[1]))));
+  for (int q = 5; q < c.nv; q++) ust[q] = R(0);
+  // sst is neither side's when it is not a number
+  const bool none = !(sst >= R(0)) && !(sst <= R(0));
+  for (int q = 0; q < c.nv; q++) ff[q] = none ? R(NAN) : fK[q] + sK * (ust[q] - uK[q]);
 }
 
 // star state of one side for HLLD (source/hlld.f90:241-257, 289-305, 337-365)

@@ -1,5 +1,5 @@
 // wx_plain.hip - the plain FP64 form: one kernel per reference routine,
-// arrays with two ghost layers per block ([blk][nv][20^3], i fastest),
+// arrays with two layers of face ghosts per block ([blk][nv][NSTORE], wx_common.h),
 // arithmetic in the reference's order (built with -ffp-contract=off).
 #include <hip/hip_runtime.h>
 
@@ -8,7 +8,11 @@
 
 namespace wx {
 
-constexpr int NIF = 17 * NC * NC;   // interfaces per direction per block used by upwindStep
+// Workgroups below which the flux and update kernel splits blocks into slabs
+// (a slab of L planes solves L + 1 z faces per column).  512 MHD blocks, whole
+// step: 1053, 1008, 963, 978 us for 512, 1024, 2048, 4096; 512 hydro blocks:
+// 610, 538, 533, 534 us; 64 hydro blocks: 85, 81, 82, 82 us.
+constexpr int WX_UPDATE_WANT = 2048;
 
 // ---------------------------------------------------------------------------
 // The device physics routines applied to arrays of records (one thread per
@@ -104,12 +108,13 @@ __global__ void __launch_bounds__(256) k_boundary(DevCfg c, double *A, int depth
   int nv = c.nv;
   double val[MAXV];
   for (int v = 0; v < nv; v++) val[v] = ghost_value<double>(A, nv, s, v);
-  for (int v = 0; v < nv; v++) A[((size_t)b * nv + v) * NCELL + q] = val[v];
+  for (int v = 0; v < nv; v++) A[((size_t)b * nv + v) * NSTORE + q] = val[v];
 }
 
 // Wind sources over interior and face-ghost cells (userBoundary).
 // grid (28, nblk): 16 blocks of 256 interior cells, 12 of face ghosts.
-__global__ void __launch_bounds__(256) k_winds(DevCfg c, double *A, PlaneWind pw) {
+// P, when given, takes the primitives of the covered interior cells.
+__global__ void __launch_bounds__(256) k_winds(DevCfg c, double *A, PlaneWind pw, double *P) {
   int b = blockIdx.y;
   int i, j, k;
   if (blockIdx.x < 16) {
@@ -129,7 +134,13 @@ __global__ void __launch_bounds__(256) k_winds(DevCfg c, double *A, PlaneWind pw
   if (plane_wind_state(c, pw, b, k, u)) hit = true;   // after the spherical sources
   if (hit) {
     int q = cid(i, j, k);
-    for (int v = 0; v < c.nv; v++) A[((size_t)b * c.nv + v) * NCELL + q] = u[v];
+    for (int v = 0; v < c.nv; v++) A[((size_t)b * c.nv + v) * NSTORE + q] = u[v];
+    if (P && blockIdx.x < 16) {
+      double p[MAXV];
+      flow2prim(c.pd, u, p);   // no passive scalars: refused with wind sources, unset by the plane wind
+      for (int v = 0; v < c.pd.nv; v++) P[((size_t)b * c.nv + v) * NSTORE + q] = p[v];
+      for (int v = c.pd.nv; v < c.nv; v++) P[((size_t)b * c.nv + v) * NSTORE + q] = u[v];
+    }
   }
 }
 
@@ -159,15 +170,70 @@ __global__ void __launch_bounds__(256) k_prims(DevCfg c, const double *A, double
     i = d[0]; j = d[1]; k = d[2];
   }
   int nv = c.nv, q = cid(i, j, k);
-  const double *Ab = A + (size_t)b * nv * NCELL;
+  const double *Ab = A + (size_t)b * nv * NSTORE;
   double u[MAXV], p[MAXV];
   if (ghost && Ab[q] == 0.0) return;
-  for (int v = 0; v < nv; v++) u[v] = Ab[v * NCELL + q];
+  for (int v = 0; v < nv; v++) u[v] = Ab[v * NSTORE + q];
   int st = flow2prim(c.pd, u, p);
   for (int v = c.pd.nv; v < nv; v++) p[v] = u[v];   // passive scalars (hydro_core.f90:372-374)
-  double *Pb = P + (size_t)b * nv * NCELL;
-  for (int v = 0; v < nv; v++) Pb[v * NCELL + q] = p[v];
+  double *Pb = P + (size_t)b * nv * NSTORE;
+  for (int v = 0; v < nv; v++) Pb[v * NSTORE + q] = p[v];
   if (st && bad && !ghost) atomicAdd(bad, 1ull);
+}
+
+// ---------------------------------------------------------------------------
+// boundary(depth) and calcPrimsAll(CELLS_GHOST) in one pass: each face ghost
+// of the first `exchange` layers is filled from its source, and the
+// primitives of both layers are formed from the value in hand (a layer that
+// was not exchanged is read; zero density is left alone, as calcPrimsAll
+// does, and then keeps the primitives of Pold).  The source of a workgroup's
+// cells is of one kind (one face of one block), so nothing diverges.  Bound:
+// the lines of the x faces, whose sources lie a row (a 128-byte line) apart;
+// both layers go to one workgroup so that it fetches each line once.
+// grid (6, nblk).
+// ---------------------------------------------------------------------------
+template <int NV, int NF>
+__global__ void __launch_bounds__(256) k_ghosts(DevCfg c, double *A, double *P, const double *Pold, int exchange) {
+  const int b = blockIdx.y, f = blockIdx.x;
+  const int a1 = threadIdx.x % NC + 1, a2 = threadIdx.x / NC + 1;
+  const int n = f >> 1;
+  Phys<double> ph = c.pd;
+  ph.nv = NF;
+#pragma unroll
+  for (int g = 1; g <= 2; g++) {
+    const int gn = (f & 1) ? NC + g : 1 - g;
+    const int q = n == 0 ? cid(gn, a1, a2) : (n == 1 ? cid(a1, gn, a2) : cid(a1, a2, gn));
+    double *Ab = A + (size_t)b * NV * NSTORE + q;
+    double *Pb = P + (size_t)b * NV * NSTORE + q;
+    double u[NV], p[NV];
+    bool have = false;
+    if (g <= exchange) {
+      GhostSrc s;
+      have = ghost_source(c.info, c.bc, b, f, g, a1, a2, s);
+      if (have) {
+#pragma unroll
+        for (int v = 0; v < NV; v++) u[v] = ghost_value<double>(A, NV, s, v);
+#pragma unroll
+        for (int v = 0; v < NV; v++) Ab[v * NSTORE] = u[v];
+      }
+    }
+    if (!have) u[0] = Ab[0];
+    if (u[0] == 0.0) {
+      if (Pold != P)
+#pragma unroll
+        for (int v = 0; v < NV; v++) Pb[v * NSTORE] = Pold[(size_t)b * NV * NSTORE + q + v * NSTORE];
+      continue;
+    }
+    if (!have) {
+#pragma unroll
+      for (int v = 1; v < NV; v++) u[v] = Ab[v * NSTORE];
+    }
+    flow2prim(ph, u, p);
+#pragma unroll
+    for (int v = NF; v < NV; v++) p[v] = u[v];
+#pragma unroll
+    for (int v = 0; v < NV; v++) Pb[v * NSTORE] = p[v];
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -224,103 +290,185 @@ __device__ inline void passive_fluxes(const Phys<double> &c, int nv, const doubl
 
 // ---------------------------------------------------------------------------
 // HLL*fluxes (hll.f90:52-167, hllc.f90:55-201, hlle.f90:54-158,
-// hlld.f90:54-158): the 3 x 17 x 16 x 16 interfaces upwindStep reads.
-// grid (3*17, nblk), block 256; F layout [blk][dim][nv][17*16*16].
+// hlld.f90:54-158) and upwindStep (source/godunov.f90:199-277) with
+// source_function (source/sources.f90:100-133: the user terms, then Powell's
+// :38-95) in one pass.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_fluxes(DevCfg c, const double *P, double *F, int order) {
-  int b = blockIdx.y;
-  int dim = blockIdx.x / 17;
-  int s = blockIdx.x % 17;          // position along dim: interface (s | s+1)
-  int a1 = threadIdx.x % NC + 1, a2 = threadIdx.x / NC + 1;
-  int n, t1, t2;
-  face_axes(2 * dim, n, t1, t2);
-  int base[3];
-  base[n] = s;
-  base[t1] = a1;
-  base[t2] = a2;
-  int nv = c.nv;
-  const double *Pb = P + (size_t)b * nv * NCELL;
-  int st = (dim == 0) ? 1 : (dim == 1) ? NB : NB * NB;
-  int q0 = cid(base[0], base[1], base[2]);
-  double pl[MAXV], pr[MAXV], ff[MAXV];
-  for (int v = 0; v < nv; v++) {
-    pl[v] = Pb[v * NCELL + q0];
-    pr[v] = Pb[v * NCELL + q0 + st];
-  }
-  swapdim(nv, dim, pl);
-  swapdim(nv, dim, pr);
-  if (order == 2) {
-    double pll[MAXV], prr[MAXV];
-    for (int v = 0; v < nv; v++) {
-      pll[v] = Pb[v * NCELL + q0 - st];
-      prr[v] = Pb[v * NCELL + q0 + 2 * st];
+// exchange of the x components of velocity and field with those along D
+template <int NV, int D> struct Turn {
+  __device__ __forceinline__ void operator()(double *v) const { swapdim(NV, D, v); }
+};
+// the same for y where d holds, per lane: selects, no branch
+template <int NV> struct TurnIf {
+  bool d;
+  __device__ __forceinline__ void operator()(double *v) const {
+    const double a = v[1], b = v[2];
+    v[1] = d ? b : a;
+    v[2] = d ? a : b;
+    if (NV == 8) {
+      const double e = v[5], f = v[6];
+      v[5] = d ? f : e;
+      v[6] = d ? e : f;
     }
-    swapdim(nv, dim, pll);
-    swapdim(nv, dim, prr);
-    for (int v = 0; v < nv; v++) limit1(pll[v], pl[v], pr[v], prr[v], c.pd.limiter);
   }
-  riemann(c.pd, pl, pr, ff);
-  if (nv > c.pd.nv) passive_fluxes(c.pd, nv, pl, pr, ff);
-  swapdim(nv, dim, ff);
-  // interface index: position s fastest along dim, then t1, then t2
-  int idx = ((a2 - 1) * NC + (a1 - 1)) * 17 + s;
-  double *Fb = F + ((size_t)b * 3 + dim) * nv * NIF;
-  for (int v = 0; v < nv; v++) Fb[(size_t)v * NIF + idx] = ff[v];
+};
+
+// cells around a face along one axis, as offsets into a block's variable
+struct Cells {
+  int ll, l, r, rr;
+};
+
+// flux between the cells l and r of one block's primitives
+template <int NV, int NF, int SOLVER, int ORDER, typename T>
+__device__ __forceinline__ void face(const Phys<double> &P, const double *Pb, const Cells &o, const T &turn,
+                                     double *ff) {
+  double pl[NV], pr[NV];
+#pragma unroll
+  for (int v = 0; v < NV; v++) {
+    pl[v] = Pb[v * NSTORE + o.l];
+    pr[v] = Pb[v * NSTORE + o.r];
+  }
+  if constexpr (ORDER == 2) {
+    double pll[NV], prr[NV];
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      pll[v] = Pb[v * NSTORE + o.ll];
+      prr[v] = Pb[v * NSTORE + o.rr];
+    }
+    limit_all<NV>(pll, pl, pr, prr, P.limiter);
+  }
+  turn(pl);
+  turn(pr);
+  if constexpr (SOLVER == SOLVER_HLLC) primfhllc_sel(P, pl, pr, ff);
+  else if constexpr (SOLVER == SOLVER_HLLD) primfhlld_sel(P, pl, pr, ff);
+  else if constexpr (SOLVER == SOLVER_HLLE) primfhlle(P, pl, pr, ff);
+  else primfhll(P, pl, pr, ff);
+  if constexpr (NV > NF) passive_fluxes(P, NV, pl, pr, ff);
+  turn(ff);
 }
 
-__device__ inline int fidx(int s, int a1, int a2) { return ((a2 - 1) * NC + (a1 - 1)) * 17 + s; }
-
-// ---------------------------------------------------------------------------
-// upwindStep (source/godunov.f90:199-277) with source_function
-// (source/sources.f90:100-133: the user terms, then Powell's :38-95).
-// grid (16, nblk).
-// ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_upwind(DevCfg c, const double *U, const double *P, const double *F,
-                                                double *UP, double dtp, UserSource us) {
-  int b = blockIdx.y;
-  int t = blockIdx.x * 256 + threadIdx.x;
-  int i = t % NC + 1, j = (t / NC) % NC + 1, k = t / (NC * NC) + 1;
-  int nv = c.nv, l = c.info[b].level - 1;
-  double dx = c.dx[0][l], dy = c.dx[1][l], dz = c.dx[2][l];
-  double dtdx = dtp / dx, dtdy = dtp / dy, dtdz = dtp / dz;
-  const double *Fx = F + ((size_t)b * 3 + 0) * nv * NIF;
-  const double *Fy = F + ((size_t)b * 3 + 1) * nv * NIF;
-  const double *Fz = F + ((size_t)b * 3 + 2) * nv * NIF;
-  int q = cid(i, j, k);
-  const double *Ub = U + (size_t)b * nv * NCELL;
-  double *UPb = UP + (size_t)b * nv * NCELL;
-  // x: (s=i, t1=j, t2=k); y: (s=j, t1=i, t2=k); z: (s=k, t1=i, t2=j)
-  int ix0 = fidx(i - 1, j, k), ix1 = fidx(i, j, k);
-  int iy0 = fidx(j - 1, i, k), iy1 = fidx(j, i, k);
-  int iz0 = fidx(k - 1, i, j), iz1 = fidx(k, i, j);
-  double upv[MAXV];
-  for (int v = 0; v < nv; v++) {
-    size_t o = (size_t)v * NIF;
-    upv[v] = Ub[v * NCELL + q] + dtdx * (Fx[o + ix0] - Fx[o + ix1]) + dtdy * (Fy[o + iy0] - Fy[o + iy1]) +
-             dtdz * (Fz[o + iz0] - Fz[o + iz1]);
-  }
-  const bool powell = c.eight_wave && nv == 8;
-  if (powell || us.on) {
-    const double *Pb = P + (size_t)b * nv * NCELL;
-    double pp[MAXV];
-    for (int v = 0; v < nv; v++) pp[v] = Pb[v * NCELL + q];
-    double s[MAXV] = {0, 0, 0, 0, 0, 0, 0, 0};
-    if (us.on) user_source(us, pp, s);
-    if (powell) {
-      double divB = (Pb[5 * NCELL + q + 1] - Pb[5 * NCELL + q - 1]) / (2.0 * dx) +
-                    (Pb[6 * NCELL + q + NB] - Pb[6 * NCELL + q - NB]) / (2.0 * dy) +
-                    (Pb[7 * NCELL + q + NB * NB] - Pb[7 * NCELL + q - NB * NB]) / (2.0 * dz);
-      s[1] = s[1] - divB * pp[5];
-      s[2] = s[2] - divB * pp[6];
-      s[3] = s[3] - divB * pp[7];
-      s[4] = s[4] - divB * (pp[1] * pp[5] + pp[2] * pp[6] + pp[3] * pp[7]);
-      s[5] = s[5] - divB * pp[1];
-      s[6] = s[6] - divB * pp[2];
-      s[7] = s[7] - divB * pp[3];
+// One workgroup updates L planes of a block; lane (i, j) owns a column.  Per
+// plane each lane solves the x face and the y face below its cell and the z
+// face above it, straight from the primitives with their ghost layers (the
+// neighbours' loads hit the L1); the 32 faces at the far ends of the rows and
+// columns go to the last 32 lanes.  x and y fluxes pass through LDS.
+//
+// Bound: FP64 issue and its latency at 3 waves per SIMD (IEEE divisions and
+// square roots of the Riemann solver, 3.1 to 4.1 solves per cell, about 3200
+// instructions per MHD cell).  512 MHD blocks (HLLD): 295 us the first stage,
+// 348 us the second; with the fluxes through HBM in a pass of their own, and
+// run-time variable counts that put the states into scratch, 1753 us each.
+// The lower z flux waits in LDS and the upper one is solved last: held in
+// registers through the x and y faces it costs a wave per SIMD.
+// P2, when given, takes the primitives of the updated interior (the next
+// stage's), so that they are not formed in a pass of their own.
+template <int NV, int NF, int SOLVER, int ORDER>
+__global__ void __launch_bounds__(256, 3)
+    k_update(DevCfg c, const double *U, const double *P, double *UP, double *P2, const StepState *ss, double dt_host,
+             int half, UserSource us, int L) {
+  constexpr int NX = NC + 1;
+  constexpr bool S2 = ORDER == 2;
+  __shared__ double sfx[NV][NC * NX];   // [v][(j-1)*17 + s]
+  __shared__ double sfy[NV][NX * NC];   // [v][s*16 + (i-1)]
+  __shared__ double sfz[NV][256];       // z flux below the lane's cell
+  const int b = blockIdx.y, k0 = blockIdx.x * L + 1, k1 = k0 + L - 1;
+  const int tid = threadIdx.x, ti = tid % NC, tj = tid / NC, i = ti + 1, j = tj + 1;
+  const int l = c.info[b].level - 1;
+  const double dt = ss ? ss->dt : dt_host;
+  const double dtp = half ? dt / 2.0 : dt;
+  const double dx = c.dx[0][l], dy = c.dx[1][l], dz = c.dx[2][l];
+  const double dtdx = dtp / dx, dtdy = dtp / dy, dtdz = dtp / dz;
+  Phys<double> ph = c.pd;
+  ph.nv = NF;
+  const double *Pb = P + (size_t)b * NV * NSTORE;
+  const double *Ub = U + (size_t)b * NV * NSTORE;
+  double *UPb = UP + (size_t)b * NV * NSTORE;
+  for (int k = k0 - 1; k <= k1; k++) {
+    if (k >= k0) {
+      {
+        double ff[NV];
+        face<NV, NF, SOLVER, ORDER>(
+            ph, Pb, Cells{S2 ? cid(i - 2, j, k) : 0, cid(i - 1, j, k), cid(i, j, k), S2 ? cid(i + 1, j, k) : 0},
+            Turn<NV, 0>{}, ff);
+        if (k > k0) __syncthreads();   // the plane below has been read
+#pragma unroll
+        for (int v = 0; v < NV; v++) sfx[v][tj * NX + ti] = ff[v];
+      }
+      {
+        double ff[NV];
+        face<NV, NF, SOLVER, ORDER>(
+            ph, Pb, Cells{S2 ? cid(i, j - 2, k) : 0, cid(i, j - 1, k), cid(i, j, k), S2 ? cid(i, j + 1, k) : 0},
+            Turn<NV, 1>{}, ff);
+#pragma unroll
+        for (int v = 0; v < NV; v++) sfy[v][tj * NC + ti] = ff[v];
+      }
+      if (tid >= 256 - 2 * NC) {
+        const bool d = tid >= 256 - NC;            // y face
+        const int aa = tid & (NC - 1);             // row or column
+        double ff[NV];
+        const int one = d ? NC : 1, last = d ? cid(aa + 1, NC, k) : cid(NC, aa + 1, k);
+        const int out = d ? cid(aa + 1, NC + 1, k) : cid(NC + 1, aa + 1, k);
+        face<NV, NF, SOLVER, ORDER>(ph, Pb, Cells{last - one, last, out, out + NC * NC}, TurnIf<NV>{d}, ff);
+#pragma unroll
+        for (int v = 0; v < NV; v++) *(d ? &sfy[v][NC * NC + aa] : &sfx[v][aa * NX + NC]) = ff[v];
+      }
     }
-    for (int v = 0; v < nv; v++) upv[v] = upv[v] + dtp * s[v];
+    // the z face last, so that its flux is not held through the others
+    double fzc[NV];
+    face<NV, NF, SOLVER, ORDER>(
+        ph, Pb, Cells{S2 ? cid(i, j, k - 1) : 0, cid(i, j, k), cid(i, j, k + 1), S2 ? cid(i, j, k + 2) : 0},
+        Turn<NV, 2>{}, fzc);
+    if (k == k0 - 1) {
+#pragma unroll
+      for (int v = 0; v < NV; v++) sfz[v][tid] = fzc[v];
+      continue;
+    }
+    __syncthreads();
+    const int q = cid(i, j, k);
+    double upv[NV];
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      upv[v] = Ub[v * NSTORE + q] + dtdx * (sfx[v][tj * NX + ti] - sfx[v][tj * NX + ti + 1]) +
+               dtdy * (sfy[v][tj * NC + ti] - sfy[v][(tj + 1) * NC + ti]) + dtdz * (sfz[v][tid] - fzc[v]);
+      sfz[v][tid] = fzc[v];
+    }
+    const bool powell = c.eight_wave && NV == 8;
+    if (powell || us.on) {
+      double pp[NV];
+#pragma unroll
+      for (int v = 0; v < NV; v++) pp[v] = Pb[v * NSTORE + q];
+      double s[MAXV] = {0, 0, 0, 0, 0, 0, 0, 0};
+      if (us.on) user_source(us, pp, s);
+      if constexpr (NV == 8) {
+        if (powell) {
+          const double *Bx = Pb + 5 * NSTORE, *By = Pb + 6 * NSTORE, *Bz = Pb + 7 * NSTORE;
+          double divB = (Bx[cid(i + 1, j, k)] - Bx[cid(i - 1, j, k)]) / (2.0 * dx) +
+                        (By[cid(i, j + 1, k)] - By[cid(i, j - 1, k)]) / (2.0 * dy) +
+                        (Bz[cid(i, j, k + 1)] - Bz[cid(i, j, k - 1)]) / (2.0 * dz);
+          s[1] = s[1] - divB * pp[5];
+          s[2] = s[2] - divB * pp[6];
+          s[3] = s[3] - divB * pp[7];
+          s[4] = s[4] - divB * (pp[1] * pp[5] + pp[2] * pp[6] + pp[3] * pp[7]);
+          s[5] = s[5] - divB * pp[1];
+          s[6] = s[6] - divB * pp[2];
+          s[7] = s[7] - divB * pp[3];
+        }
+      }
+#pragma unroll
+      for (int v = 0; v < NV; v++) upv[v] = upv[v] + dtp * s[v];
+    }
+#pragma unroll
+    for (int v = 0; v < NV; v++) UPb[v * NSTORE + q] = upv[v];
+    if (P2) {
+      double p[NV];
+      flow2prim(ph, upv, p);
+#pragma unroll
+      for (int v = NF; v < NV; v++) p[v] = upv[v];   // passive scalars (hydro_core.f90:372-374)
+      double *P2b = P2 + (size_t)b * NV * NSTORE;
+#pragma unroll
+      for (int v = 0; v < NV; v++) P2b[v * NSTORE + q] = p[v];
+    }
   }
-  for (int v = 0; v < nv; v++) UPb[v * NCELL + q] = upv[v];
 }
 
 // ---------------------------------------------------------------------------
@@ -331,45 +479,72 @@ __global__ void __launch_bounds__(256) k_viscous(DevCfg c, const double *UP, dou
   int t = blockIdx.x * 256 + threadIdx.x;
   int i = t % NC + 1, j = (t / NC) % NC + 1, k = t / (NC * NC) + 1;
   int q = cid(i, j, k);
+  const int xp = cid(i + 1, j, k), xm = cid(i - 1, j, k), yp = cid(i, j + 1, k), ym = cid(i, j - 1, k),
+            zp = cid(i, j, k + 1), zm = cid(i, j, k - 1);
   double eta = c.visc_eta;
   for (int v = 0; v < c.nv; v++) {
-    const double *A = UP + ((size_t)b * c.nv + v) * NCELL;
-    U[((size_t)b * c.nv + v) * NCELL + q] =
-        A[q] + eta * (+A[q + 1] + A[q - 1] + A[q + NB] + A[q - NB] + A[q + NB * NB] + A[q - NB * NB] - 6.0 * A[q]);
+    const double *A = UP + ((size_t)b * c.nv + v) * NSTORE;
+    U[((size_t)b * c.nv + v) * NSTORE + q] =
+        A[q] + eta * (+A[xp] + A[xm] + A[yp] + A[ym] + A[zp] + A[zm] - 6.0 * A[q]);
   }
 }
 
 // ---------------------------------------------------------------------------
 // getTimestep (source/hydro_solver.f90:129-211): min over interior cells.
 // Positive doubles order like their bit patterns, so the global minimum is
-// an unsigned 64-bit atomicMin on the bits.  grid (16, nblk).
+// an unsigned 64-bit atomicMin on the bits.  One workgroup and one atomic per
+// block, over DT_SLOTS words that the reader folds: atomics on one word are
+// served one after the other, about 12 ns each, and one per wavefront of 64
+// cells cost more than the pass itself (386 us for 512 MHD blocks).
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_timestep(DevCfg c, const double *P, unsigned long long *dtbits) {
-  int b = blockIdx.y;
-  int t = blockIdx.x * 256 + threadIdx.x;
-  int i = t % NC + 1, j = (t / NC) % NC + 1, k = t / (NC * NC) + 1;
-  int nv = c.nv, l = c.info[b].level - 1;
-  const double *Pb = P + (size_t)b * nv * NCELL;
-  int q = cid(i, j, k);
-  double p[MAXV];
-  for (int v = 0; v < nv; v++) p[v] = Pb[v * NCELL + q];
+template <int NV>
+__device__ __forceinline__ double dt_of(const DevCfg &c, const double *p, double dx, double dy, double dz) {
   double dt = 1.0e30;
-  if (c.pd.mhd && nv == 8) {
+  if (NV == 8 && c.pd.mhd) {
     double cfx = cfast1(c.pd, p[4], p[0], p[5], p[6], p[7], p[5]);
     double cfy = cfast1(c.pd, p[4], p[0], p[5], p[6], p[7], p[6]);
     double cfz = cfast1(c.pd, p[4], p[0], p[5], p[6], p[7], p[7]);
-    dt = fmin(dt, c.dx[0][l] / (fabs(p[1]) + cfx));
-    dt = fmin(dt, c.dx[1][l] / (fabs(p[2]) + cfy));
-    dt = fmin(dt, c.dx[2][l] / (fabs(p[3]) + cfz));
+    dt = fmin(dt, dx / (fabs(p[1]) + cfx));
+    dt = fmin(dt, dy / (fabs(p[2]) + cfy));
+    dt = fmin(dt, dz / (fabs(p[3]) + cfz));
   } else {
     double cs = sound(c.pd, p);
-    dt = fmin(dt, c.dx[0][l] / (fabs(p[1]) + cs));
-    dt = fmin(dt, c.dx[1][l] / (fabs(p[2]) + cs));
-    dt = fmin(dt, c.dx[2][l] / (fabs(p[3]) + cs));
+    dt = fmin(dt, dx / (fabs(p[1]) + cs));
+    dt = fmin(dt, dy / (fabs(p[2]) + cs));
+    dt = fmin(dt, dz / (fabs(p[3]) + cs));
   }
-  // wavefront min, then one atomic per wavefront
+  return dt;
+}
+
+// the smallest dt of a workgroup of 256 lanes into a slot
+__device__ __forceinline__ void dt_to_slot(double dt, int slot, unsigned long long *slots) {
+  __shared__ double part[4];
   for (int off = 32; off > 0; off >>= 1) dt = fmin(dt, __shfl_xor(dt, off));
-  if ((threadIdx.x & 63) == 0) atomicMin(dtbits, (unsigned long long)__double_as_longlong(dt));
+  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = dt;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    dt = fmin(fmin(part[0], part[1]), fmin(part[2], part[3]));
+    atomicMin(&slots[(slot % DT_SLOTS) * DT_STRIDE], (unsigned long long)__double_as_longlong(dt));
+  }
+}
+
+template <int NV>
+__global__ void __launch_bounds__(256) k_timestep(DevCfg c, const double *P, unsigned long long *slots) {
+  const int b = blockIdx.x, l = c.info[b].level - 1;
+  const int i = threadIdx.x % NC + 1, j = threadIdx.x / NC + 1;
+  const double dx = c.dx[0][l], dy = c.dx[1][l], dz = c.dx[2][l];
+  constexpr int NP = NV == 8 ? 8 : 5;   // passive scalars don't enter
+  const double *Pb = P + (size_t)b * NV * NSTORE;
+  double dt = 1.0e30;
+#pragma unroll 2
+  for (int k = 1; k <= NC; k++) {
+    const int q = cid(i, j, k);
+    double p[MAXV];
+#pragma unroll
+    for (int v = 0; v < NP; v++) p[v] = Pb[v * NSTORE + q];
+    dt = fmin(dt, dt_of<NV>(c, p, dx, dy, dz));
+  }
+  dt_to_slot(dt, b, slots);
 }
 
 // ---------------------------------------------------------------------------
@@ -380,19 +555,131 @@ __global__ void __launch_bounds__(256) k_cooling(DevCfg c, double *U, double *P,
   int t = blockIdx.x * 256 + threadIdx.x;
   int i = t % NC + 1, j = (t / NC) % NC + 1, k = t / (NC * NC) + 1;
   int nv = c.nv, q = cid(i, j, k);
-  double *Pb = P + (size_t)b * nv * NCELL;
+  double *Pb = P + (size_t)b * nv * NSTORE;
   double pr[5];
-  for (int v = 0; v < 5; v++) pr[v] = Pb[v * NCELL + q];
+  for (int v = 0; v < 5; v++) pr[v] = Pb[v * NSTORE + q];
   // EOS_H_RATE (calcTemp, hydro_core.f90:258-264): P = (n_HI + n_HII) k T
   // with the neutral hydrogen density in the first passive scalar
   const bool hrate = c.eos == 3;
   double th = 0.0;
-  if (hrate) th = pr[4] / (2.0 * pr[0] / mu0 - Pb[5 * NCELL + q]) * c.p_sc / KB;
+  if (hrate) th = pr[4] / (2.0 * pr[0] / mu0 - Pb[5 * NSTORE + q]) * c.p_sc / KB;
   double e;
   if (cool_cell(c, dt, pr, &e, hrate, th)) {
-    Pb[4 * NCELL + q] = pr[4];
-    U[((size_t)b * nv + 4) * NCELL + q] = e;
+    Pb[4 * NSTORE + q] = pr[4];
+    U[((size_t)b * nv + 4) * NSTORE + q] = e;
   }
+}
+
+// ---------------------------------------------------------------------------
+// The end of a step in one pass: doViscousStep (source/hydro_solver.f90:
+// 217-250), updatePrims (source/hydro_core.f90:43-59), cooling
+// (source/cooling.f90:37-118) and, with slots, getTimestep of the new state.
+// The lane of column (i, j) walks L planes and keeps the planes around k in
+// registers, so a cell of UP is read once from its column and four times by
+// its row and plane (L1).  The last 12 nblk workgroups form the primitives of
+// the face ghosts, as updatePrims does; they come after all others, so that
+// every chiplet (workgroups are dealt to them in turn) gets its share of the
+// interior.  grid (16/L + 12) nblk.
+// ---------------------------------------------------------------------------
+template <int NV, int NF>
+__global__ void __launch_bounds__(256) k_finish(DevCfg c, const double *UP, double *U, double *P,
+                                                StepState *ss, double mu0, unsigned long long *slots, int L) {
+  const int ns = NC / L, slab = blockIdx.x % ns;
+  const bool inside = (int)blockIdx.x < c.nblk * ns;
+  const int gw = (int)blockIdx.x - c.nblk * ns;
+  const int b = inside ? blockIdx.x / ns : gw / 12;
+  Phys<double> ph = c.pd;
+  ph.nv = NF;
+  double *Ub = U + (size_t)b * NV * NSTORE, *Pb = P + (size_t)b * NV * NSTORE;
+  if (!inside) {
+    const int e = gw % 12, f = e >> 1, g = (e & 1) + 1;
+    const int a1 = threadIdx.x % NC + 1, a2 = threadIdx.x / NC + 1;
+    const int n = f >> 1, gn = (f & 1) ? NC + g : 1 - g;
+    const int q = n == 0 ? cid(gn, a1, a2) : (n == 1 ? cid(a1, gn, a2) : cid(a1, a2, gn));
+    double u[NV], p[NV];
+    u[0] = Ub[q];
+    if (u[0] == 0.0) return;
+#pragma unroll
+    for (int v = 1; v < NV; v++) u[v] = Ub[v * NSTORE + q];
+    flow2prim(ph, u, p);
+#pragma unroll
+    for (int v = NF; v < NV; v++) p[v] = u[v];
+#pragma unroll
+    for (int v = 0; v < NV; v++) Pb[v * NSTORE + q] = p[v];
+    return;
+  }
+  const int l = c.info[b].level - 1;
+  const double dx = c.dx[0][l], dy = c.dx[1][l], dz = c.dx[2][l];
+  const int i = threadIdx.x % NC + 1, j = threadIdx.x / NC + 1, k0 = slab * L + 1;
+  const double eta = c.visc_eta, dt = ss->dt;
+  const double *A = UP + (size_t)b * NV * NSTORE;
+  double below[NV], here[NV], dtmin = 1.0e30;
+  int floors = 0;
+#pragma unroll
+  for (int v = 0; v < NV; v++) {
+    below[v] = A[v * NSTORE + cid(i, j, k0 - 1)];
+    here[v] = A[v * NSTORE + cid(i, j, k0)];
+  }
+  for (int k = k0; k < k0 + L; k++) {
+    const int q = cid(i, j, k), xp = cid(i + 1, j, k), xm = cid(i - 1, j, k), yp = cid(i, j + 1, k),
+              ym = cid(i, j - 1, k), zp = cid(i, j, k + 1);
+    double u[NV], p[NV], above[NV];
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      const double *a = A + v * NSTORE;
+      above[v] = a[zp];
+      u[v] = here[v] + eta * (+a[xp] + a[xm] + a[yp] + a[ym] + above[v] + below[v] - 6.0 * here[v]);
+    }
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      below[v] = here[v];
+      here[v] = above[v];
+    }
+    if (flow2prim(ph, u, p)) floors++;
+#pragma unroll
+    for (int v = NF; v < NV; v++) p[v] = u[v];   // passive scalars (hydro_core.f90:372-374)
+    if (c.cooling) {
+      double e, th = 0.0;
+      const bool hrate = NV > NF && c.eos == 3;
+      if constexpr (NV > NF) {
+        if (hrate) th = p[4] / (2.0 * p[0] / mu0 - p[5]) * c.p_sc / KB;   // see k_cooling
+      }
+      if (cool_cell(c, dt, p, &e, hrate, th)) u[4] = e;
+    }
+#pragma unroll
+    for (int v = 0; v < NV; v++) {
+      Ub[v * NSTORE + q] = u[v];
+      Pb[v * NSTORE + q] = p[v];
+    }
+    if (slots) dtmin = fmin(dtmin, dt_of<NV>(c, p, dx, dy, dz));
+  }
+  if (floors) atomicAdd(&ss->floors, (unsigned long long)floors);
+  if (slots) dt_to_slot(dtmin, blockIdx.x, slots);
+}
+
+// The scalars of a step: closes the step before it (advance), then dt from
+// the smallest of the slots with the start-up ramp and the output clamp
+// (source/hydro_solver.f90:183-207).  The slots are cleared for the next
+// reduction.  One wavefront.
+__global__ void __launch_bounds__(64) k_step_begin(StepState *s, unsigned long long *slots, double cfl, int cooling,
+                                                   int advance) {
+  static_assert(DT_SLOTS == 64, "one slot per lane");
+  double m = __longlong_as_double((long long)slots[threadIdx.x * DT_STRIDE]);
+  slots[threadIdx.x * DT_STRIDE] = ~0ull;
+  // an untouched slot reads as a NaN, which fmin drops
+  for (int off = 32; off > 0; off >>= 1) m = fmin(m, __shfl_xor(m, off));
+  if (threadIdx.x == 0) {
+    if (advance) step_close(s);
+    step_open(s, m, cfl, cooling);
+  }
+}
+
+// the smallest of the slots into *out, the slots cleared
+__global__ void __launch_bounds__(64) k_dt_fold(unsigned long long *slots, unsigned long long *out) {
+  double m = __longlong_as_double((long long)slots[threadIdx.x * DT_STRIDE]);
+  slots[threadIdx.x * DT_STRIDE] = ~0ull;
+  for (int off = 32; off > 0; off >>= 1) m = fmin(m, __shfl_xor(m, off));
+  if (threadIdx.x == 0) *out = (unsigned long long)__double_as_longlong(m);
 }
 
 // ---------------------------------------------------------------------------
@@ -412,13 +699,13 @@ __global__ void __launch_bounds__(256) k_mark(DevCfg c, const double *P, double 
   const double two_dx = 2.0 * c.dx[0][c.info[b].level - 1];
   double m = 0.0;
   for (int s = 0; s < 2; s++) {
-    const double *A = P + ((size_t)b * c.nv + (s == 0 ? 4 : 0)) * NCELL;
+    const double *A = P + ((size_t)b * c.nv + (s == 0 ? 4 : 0)) * NSTORE;
     for (int k = 1; k <= NC; k++) {
       const int q = cid(i, j, k);
       const double a = A[q];
-      const double gx = fabs(A[q + 1] - A[q - 1]) / a / two_dx;
-      const double gy = fabs(A[q + NB] - A[q - NB]) / a / two_dx;
-      const double gz = fabs(A[q + NB * NB] - A[q - NB * NB]) / a / two_dx;
+      const double gx = fabs(A[cid(i + 1, j, k)] - A[cid(i - 1, j, k)]) / a / two_dx;
+      const double gy = fabs(A[cid(i, j + 1, k)] - A[cid(i, j - 1, k)]) / a / two_dx;
+      const double gz = fabs(A[cid(i, j, k + 1)] - A[cid(i, j, k - 1)]) / a / two_dx;
       m = fmax(m, fmax(gx, fmax(gy, gz)));
     }
   }
@@ -541,26 +828,98 @@ __global__ void __launch_bounds__(1024) k_mark_fused(DevCfg c, const double *U, 
 // ---------------------------------------------------------------------------
 // host launchers
 // ---------------------------------------------------------------------------
+// planes per workgroup: whole columns once the mesh alone gives `want`
+// workgroups, thinner slabs below that
+static int planes_for(int nblk, int want) {
+  int L = NC;
+  while (L > 1 && nblk * (NC / L) < want) L >>= 1;
+  return L;
+}
+
+// stored variables (with passive scalars) and flow variables as constants
+#define WX_BY_NV(nv, CALL)                     \
+  do {                                         \
+    switch (nv) {                              \
+      case 5: { CALL(5, 5); break; }           \
+      case 6: { CALL(6, 5); break; }           \
+      case 7: { CALL(7, 5); break; }           \
+      default: { CALL(8, 8); break; }          \
+    }                                          \
+  } while (0)
+
 void plain_boundary(const DevCfg &c, const PlaneWind &pw, double *A, int depth, hipStream_t st) {
   hipLaunchKernelGGL(k_boundary, dim3(6 * depth, c.nblk), dim3(256), 0, st, c, A, depth);
-  if (c.nwind > 0 || pw.plane != 0) hipLaunchKernelGGL(k_winds, dim3(28, c.nblk), dim3(256), 0, st, c, A, pw);
+  double *none = nullptr;
+  if (c.nwind > 0 || pw.plane != 0) hipLaunchKernelGGL(k_winds, dim3(28, c.nblk), dim3(256), 0, st, c, A, pw, none);
+}
+void plain_ghosts(const DevCfg &c, const PlaneWind &pw, double *A, double *P, const double *Pold, int depth,
+                  double *Pcover, hipStream_t st) {
+  int exchange = depth;
+  if (c.nwind > 0 || pw.plane != 0) {
+    // a source covers ghosts too: it comes between the exchange and the primitives
+    hipLaunchKernelGGL(k_boundary, dim3(6 * depth, c.nblk), dim3(256), 0, st, c, A, depth);
+    hipLaunchKernelGGL(k_winds, dim3(28, c.nblk), dim3(256), 0, st, c, A, pw, Pcover);
+    exchange = 0;
+  }
+#define WX_CALL(NV, NF) \
+  hipLaunchKernelGGL((k_ghosts<NV, NF>), dim3(6, c.nblk), dim3(256), 0, st, c, A, P, Pold, exchange)
+  WX_BY_NV(c.nv, WX_CALL);
+#undef WX_CALL
 }
 void plain_prims(const DevCfg &c, const double *A, double *P, int cells, unsigned long long *bad,
                  hipStream_t st) {
   hipLaunchKernelGGL(k_prims, dim3(28, c.nblk), dim3(256), 0, st, c, A, P, cells, bad);
 }
-void plain_fluxes(const DevCfg &c, const double *P, double *F, int order, hipStream_t st) {
-  hipLaunchKernelGGL(k_fluxes, dim3(3 * 17, c.nblk), dim3(256), 0, st, c, P, F, order);
+
+template <int NV, int NF, int SOLVER>
+static void launch_update(const DevCfg &c, const UserSource &us, const double *U, const double *P, double *UP,
+                          double *P2, const StepState *ss, double dt, int half, int order, hipStream_t st) {
+  const int L = planes_for(c.nblk, WX_UPDATE_WANT);
+  const dim3 grid(NC / L, c.nblk);
+  if (order == 2)
+    hipLaunchKernelGGL((k_update<NV, NF, SOLVER, 2>), grid, dim3(256), 0, st, c, U, P, UP, P2, ss, dt, half, us, L);
+  else
+    hipLaunchKernelGGL((k_update<NV, NF, SOLVER, 1>), grid, dim3(256), 0, st, c, U, P, UP, P2, ss, dt, half, us, L);
 }
-void plain_upwind(const DevCfg &c, const UserSource &us, const double *U, const double *P, const double *F,
-                  double *UP, double dtp, hipStream_t st) {
-  hipLaunchKernelGGL(k_upwind, dim3(16, c.nblk), dim3(256), 0, st, c, U, P, F, UP, dtp, us);
+
+void plain_update(const DevCfg &c, const UserSource &us, const double *U, const double *P, double *UP, double *P2,
+                  const StepState *ss, double dt, int half, int order, hipStream_t st) {
+  const int solver = c.pd.solver;
+  if (c.nv == 8 && solver == SOLVER_HLLD)
+    return launch_update<8, 8, SOLVER_HLLD>(c, us, U, P, UP, P2, ss, dt, half, order, st);
+  if (c.nv == 8 && solver == SOLVER_HLLE)
+    return launch_update<8, 8, SOLVER_HLLE>(c, us, U, P, UP, P2, ss, dt, half, order, st);
+#define WX_CALL(NV, NF)                                                                            \
+  if (solver == SOLVER_HLLC) launch_update<NV, NF, SOLVER_HLLC>(c, us, U, P, UP, P2, ss, dt, half, order, st); \
+  else launch_update<NV, NF, SOLVER_HLL>(c, us, U, P, UP, P2, ss, dt, half, order, st)
+  WX_BY_NV(c.nv, WX_CALL);
+#undef WX_CALL
 }
 void plain_viscous(const DevCfg &c, const double *UP, double *U, hipStream_t st) {
   hipLaunchKernelGGL(k_viscous, dim3(16, c.nblk), dim3(256), 0, st, c, UP, U);
 }
-void plain_timestep(const DevCfg &c, const double *P, unsigned long long *dtbits, hipStream_t st) {
-  hipLaunchKernelGGL(k_timestep, dim3(16, c.nblk), dim3(256), 0, st, c, P, dtbits);
+void plain_finish(const DevCfg &c, const double *UP, double *U, double *P, StepState *ss, double mu0,
+                  unsigned long long *slots, hipStream_t st) {
+  const int L = planes_for(c.nblk, 2048);
+#define WX_CALL(NV, NF)                                                                                          \
+  hipLaunchKernelGGL((k_finish<NV, NF>), dim3((NC / L + 12) * c.nblk), dim3(256), 0, st, c, UP, U, P, ss, mu0, slots, L)
+  WX_BY_NV(c.nv, WX_CALL);
+#undef WX_CALL
+}
+static void launch_timestep(const DevCfg &c, const double *P, unsigned long long *slots, hipStream_t st) {
+#define WX_CALL(NV, NF) hipLaunchKernelGGL(k_timestep<NV>, dim3(c.nblk), dim3(256), 0, st, c, P, slots)
+  WX_BY_NV(c.nv, WX_CALL);
+#undef WX_CALL
+}
+void plain_timestep(const DevCfg &c, const double *P, unsigned long long *slots, unsigned long long *dtbits,
+                    hipStream_t st) {
+  launch_timestep(c, P, slots, st);
+  hipLaunchKernelGGL(k_dt_fold, dim3(1), dim3(64), 0, st, slots, dtbits);
+}
+void plain_step_begin(const DevCfg &c, const double *P, StepState *ss, unsigned long long *slots, int advance,
+                      hipStream_t st) {
+  if (P) launch_timestep(c, P, slots, st);
+  hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(64), 0, st, ss, slots, c.cfl, c.cooling, advance);
 }
 void plain_cooling(const DevCfg &c, double *U, double *P, double dt, double mu0, hipStream_t st) {
   hipLaunchKernelGGL(k_cooling, dim3(16, c.nblk), dim3(256), 0, st, c, U, P, dt, mu0);
@@ -574,6 +933,5 @@ void fused_ghost_prims(const DevCfg &c, const double *U, double *G, hipStream_t 
 void fused_mark(const DevCfg &c, const double *U, const double *G, double *maxgrad, hipStream_t st) {
   hipLaunchKernelGGL(k_mark_fused, dim3(c.nblk), dim3(1024), 0, st, c, U, G, maxgrad);
 }
-size_t plain_flux_elems(int nblk, int nv) { return (size_t)nblk * 3 * nv * NIF; }
 
 }  // namespace wx
