@@ -530,7 +530,7 @@ int plain_steps(Ctx *c, int nsteps, int *it, double *dt, double *time, int *next
   s.t_sc = t_sc;
   HIPCHK(hipMemcpyAsync(c->d_ss, &s, sizeof(s), hipMemcpyHostToDevice, c->st));
   for (int n = 0; n < nsteps; n++) {
-    plain_step_begin(c->dc, n == 0 ? c->dP : nullptr, c->d_ss, c->d_slots, n > 0, c->st);
+    plain_step_begin(c->dc, n == 0 ? c->dP : nullptr, c->d_ss, c->d_slots, c->st);
     plain_stages(c, c->cfg.solver == SOLVER_HLL1 ? 1 : 2, c->d_ss, 0.0);
     plain_finish(c->dc, c->dUP, c->dU, c->dP, c->d_ss, c->cfg.mu0, n + 1 < nsteps ? c->d_slots : nullptr, c->st);
   }

@@ -43,12 +43,11 @@ struct StepState {
   int it;             // iteration counter
   int nextout;        // next output number
   int dump;           // the clamp fired this step
-  int pad;
+  int open;           // the step's time is still to be added (step_close)
   unsigned long long floors;      // cells floored in the current step (plain form)
 };
 
-// words over which workgroups spread the smallest dt of the plain form (one
-// per 64-byte line)
+// words over which workgroups spread the smallest dt (one per 64-byte line)
 constexpr int DT_SLOTS = 64, DT_STRIDE = 8;
 
 // dt of a step from the smallest dx/(|v|+c): CFL, start-up ramp, output
@@ -66,11 +65,24 @@ __device__ inline void step_open(StepState *s, double m, double cfl, int cooling
   }
   s->dt = dtl;
   s->floors = 0;
+  s->open = 1;
 }
 
 __host__ __device__ inline void step_close(StepState *s) {
+  if (!s->open) return;
+  s->open = 0;
   s->time = s->time + s->dt;
   if (s->dump) s->nextout += 1;
+}
+
+// One wavefront: the smallest of the slots, which are cleared.  An untouched
+// slot reads as a NaN, which fmin drops.
+__device__ __forceinline__ double fold_slots(unsigned long long *slots) {
+  static_assert(DT_SLOTS == 64, "one slot per lane");
+  double m = __longlong_as_double((long long)slots[threadIdx.x * DT_STRIDE]);
+  slots[threadIdx.x * DT_STRIDE] = ~0ull;
+  for (int off = 32; off > 0; off >>= 1) m = fmin(m, __shfl_xor(m, off));
+  return m;
 }
 
 // ---------------------------------------------------------------------------

@@ -18,6 +18,9 @@ struct FusedState {
   // into this second buffer, and the two swap roles every step
   double *U2 = nullptr;
   int two_u = 0;
+  // hydro: the state between the second stage and the end of the step
+  double *X = nullptr;
+  unsigned long long *slots = nullptr;   // partial minima of dt, next to step's dtmin_bits
   void *UP = nullptr;        // [blk][nv][4096] half-step state (FP32, or FP64 in the fp64 variant)
   int fp64 = 0;              // flux arithmetic and UP storage in FP64
   int *order = nullptr;      // block processing order (device)
@@ -27,7 +30,7 @@ struct FusedState {
   int xcd_map = 1;           // XCD-aware block order
   int curve = 0;             // block order along the Morton (0) or Hilbert (1) curve
   int mhd_plain32 = 0;       // FP32 MHD: plain FP32 fluxes (1) instead of the delta form (0)
-  int nslab = 1;             // FP32 MHD without viscosity: z slabs per block, one workgroup each
+  int nslab = 0;             // z slabs per block where set_tuning chose them, 0: by mesh size
   int nroot[3] = {1, 1, 1};  // root blocks per axis (Hilbert curve order)
   hipGraph_t graph = nullptr;      // one step from the current U
   hipGraphExec_t exec = nullptr;

@@ -27,8 +27,17 @@
 #include "wx_fused.h"
 #include "wx_hilbert.h"
 #include "wx_fused_kern.h"
+#include "wx_hydro_kern.h"
 
 namespace wx {
+
+// Workgroups below which the hydro kernels take thinner slabs (a slab of L
+// planes solves L + 1 z faces and loads L + 3 planes per column).  us per step
+// for HYDRO_WANT = 512, 1024, 2048, 4096: 64 blocks 58.9, 56.1, 56.3, 55.5; 904
+// blocks on 4 levels 519, 478, 466, 472; 1728 blocks 759, 758, 749, 761.  The
+// end of the step runs 4 planes per workgroup, fewer below END_WANT: 64 blocks
+// 52.6, 56.1, 55.6 for 512, 1024, 2048.
+constexpr int HYDRO_WANT = 2048, END_WANT = 512;
 
 static thread_local std::string f_err;
 const char *fused_error() { return f_err.c_str(); }
@@ -50,14 +59,19 @@ __global__ void __launch_bounds__(256) k_dt_init(FusedArgs a) {
   if ((threadIdx.x & 63) == 0) atomicMin(&a.step->dtmin_bits, (unsigned long long)__double_as_longlong(m));
 }
 
-// dt of the step: CFL, start-up ramp, output clamp
-// (source/hydro_solver.f90:183-207); resets the running minimum
-__global__ void k_dt_finalize(StepState *s, double cfl, int cooling) {
-  step_open(s, __longlong_as_double((long long)s->dtmin_bits), cfl, cooling);
-  s->dtmin_bits = ~0ull;
+// The scalars of a step: closes the step before it, then dt from the running
+// minimum (the kernels' slots and the step record's own word) with the
+// start-up ramp and the output clamp (source/hydro_solver.f90:183-207); both
+// minima are cleared.  One wavefront.
+__global__ void __launch_bounds__(64) k_begin(StepState *s, unsigned long long *slots, double cfl, int cooling) {
+  double m = fold_slots(slots);
+  if (threadIdx.x == 0) {
+    m = fmin(m, __longlong_as_double((long long)s->dtmin_bits));
+    step_close(s);
+    step_open(s, m, cfl, cooling);
+    s->dtmin_bits = ~0ull;
+  }
 }
-
-__global__ void k_step_post(StepState *s) { step_close(s); }
 
 // PRIM of the state in the same layout ([blk][nv][16^3]), for downloads
 template <int NV>
@@ -141,6 +155,8 @@ int fused_alloc(FusedState &f, const DevCfg &c, const std::vector<BlockInfo> &in
   FCHK(hipMalloc(&f.UP, n * (f.fp64 ? sizeof(double) : sizeof(float))));
   FCHK(hipMalloc(&f.order, c.nblk * sizeof(int)));
   FCHK(hipMalloc(&f.step, sizeof(StepState)));
+  if (c.nv == 5) FCHK(hipMalloc(&f.X, n * sizeof(double)));
+  FCHK(hipMalloc(&f.slots, DT_SLOTS * DT_STRIDE * sizeof(unsigned long long)));
   f.host_info = info;
   f.maxlev = c.maxlev;
   if (build_order(f)) return 1;
@@ -166,6 +182,8 @@ void fused_free(FusedState &f) {
   hipFree(f.UP);
   hipFree(f.order);
   hipFree(f.step);
+  hipFree(f.X);
+  hipFree(f.slots);
   for (int e = 0; e < 4; e++)
     if (f.ev[e]) hipEventDestroy(f.ev[e]);
   for (int e = 0; e < 4; e++) f.ev[e] = nullptr;
@@ -174,6 +192,8 @@ void fused_free(FusedState &f) {
   f.UP = nullptr;
   f.order = nullptr;
   f.step = nullptr;
+  f.X = nullptr;
+  f.slots = nullptr;
 }
 
 static FusedArgs make_args(FusedState &f, const DevCfg &c) {
@@ -183,6 +203,8 @@ static FusedArgs make_args(FusedState &f, const DevCfg &c) {
   a.Uout = f.U2 ? f.U2 : f.U;
   a.UPin = f.UP;
   a.UPout = f.UP;
+  a.X = f.X;
+  a.slots = f.slots;
   a.order = f.order;
   a.step = f.step;
   a.nblk = f.nblk;
@@ -206,6 +228,7 @@ int fused_upload(FusedState &f, const DevCfg &c, double *U, bool adopt, hipStrea
   StepState s{};
   s.dtmin_bits = ~0ull;
   FCHK(hipMemcpyAsync(f.step, &s, sizeof(s), hipMemcpyHostToDevice, st));
+  FCHK(hipMemsetAsync(f.slots, 0xFF, DT_SLOTS * DT_STRIDE * sizeof(unsigned long long), st));
   launch_dt_init(f, c, st);
   FCHK(hipGetLastError());
   FCHK(hipStreamSynchronize(st));
@@ -225,47 +248,100 @@ int fused_prims(FusedState &f, const DevCfg &c, double *P, hipStream_t st) {
 
 int fused_timestep(FusedState &f, const DevCfg &c, hipStream_t st, double *dt_raw) {
   StepState s;
+  unsigned long long slots[DT_SLOTS * DT_STRIDE];
   FCHK(hipMemcpyAsync(&s, f.step, sizeof(s), hipMemcpyDeviceToHost, st));
+  FCHK(hipMemcpyAsync(slots, f.slots, sizeof(slots), hipMemcpyDeviceToHost, st));
   FCHK(hipStreamSynchronize(st));
-  double m;
+  // an untouched word reads as a NaN, which fmin drops
+  double m, q;
   std::memcpy(&m, &s.dtmin_bits, sizeof(m));
+  for (int n = 0; n < DT_SLOTS; n++) {
+    std::memcpy(&q, &slots[n * DT_STRIDE], sizeof(q));
+    m = std::fmin(m, q);
+  }
   *dt_raw = c.cooling ? std::fmin(m, 1.0e30) * c.cfl : m * c.cfl;
   return 0;
 }
 
+// FP64 MHD stages, and the FP32 MHD forms
+static void launch_stage_mhd(const FusedState &f, const FusedArgs &a, int grid, int solver, bool visc, int stage,
+                             hipStream_t st) {
+  if (!f.fp64) launch_stage_mhd32(a, grid, solver, visc, stage, f.mhd_plain32, st);
+  else if (solver == SOLVER_HLLD) launch_stage_s<double, double, 8, SOLVER_HLLD>(a, grid, visc, stage, st);
+  else launch_stage_s<double, double, 8, SOLVER_HLLE>(a, grid, visc, stage, st);
+}
+
+// meshes without wind sources take kernels without the wind code; minmod, the
+// default limiter, is fixed at compile time, the others are read at run time
+template <typename RF, typename ST, int SOLVER, bool WINDS>
+static void launch_hydro_t(const FusedArgs &a, int grid, int stage, hipStream_t st) {
+  constexpr int MM = 1;   // LIMITER_MINMOD (source/constants.f90)
+  if (stage == 1)
+    hipLaunchKernelGGL((k_hydro<false, RF, ST, SOLVER, MM, WINDS>), dim3(grid), dim3(256), 0, st, a);
+  else if (a.c.pf.limiter == MM)
+    hipLaunchKernelGGL((k_hydro<true, RF, ST, SOLVER, MM, WINDS>), dim3(grid), dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL((k_hydro<true, RF, ST, SOLVER, LIM_RUNTIME, WINDS>), dim3(grid), dim3(256), 0, st, a);
+}
+
 template <typename RF, typename ST>
-static void launch_stage_t(const FusedArgs &a, int grid, int nv, int solver, bool visc, int stage, int plain32,
-                           hipStream_t st) {
-  if (nv == 8) {
-    if constexpr (sizeof(RF) == 4) {
-      launch_stage_mhd32(a, grid, solver, visc, stage, plain32, st);
-    } else {
-      if (solver == SOLVER_HLLD) launch_stage_s<RF, ST, 8, SOLVER_HLLD>(a, grid, visc, stage, st);
-      else launch_stage_s<RF, ST, 8, SOLVER_HLLE>(a, grid, visc, stage, st);
-    }
+static void launch_hydro(const FusedArgs &a, int grid, int stage, hipStream_t st) {
+  const bool winds = a.c.nwind > 0;
+  if (a.c.pd.solver == SOLVER_HLLC) {
+    if (winds) launch_hydro_t<RF, ST, SOLVER_HLLC, true>(a, grid, stage, st);
+    else launch_hydro_t<RF, ST, SOLVER_HLLC, false>(a, grid, stage, st);
   } else {
-    if (solver == SOLVER_HLLC) launch_stage_s<RF, ST, 5, SOLVER_HLLC>(a, grid, visc, stage, st);
-    else launch_stage_s<RF, ST, 5, SOLVER_HLL>(a, grid, visc, stage, st);
+    if (winds) launch_hydro_t<RF, ST, SOLVER_HLL, true>(a, grid, stage, st);
+    else launch_hydro_t<RF, ST, SOLVER_HLL, false>(a, grid, stage, st);
   }
+}
+
+template <typename RF, typename ST>
+static void launch_end(const FusedArgs &a, hipStream_t st) {
+  const int grid = a.nblk * a.nslab;
+  if (a.c.visc_eta == 0.0)
+    hipLaunchKernelGGL((k_end<5, RF, ST, false, false, false>), dim3(grid), dim3(256), 0, st, a);
+  else if (a.c.nwind > 0)
+    hipLaunchKernelGGL((k_end<5, RF, ST, true, false, true>), dim3(grid), dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL((k_end<5, RF, ST, true, false, false>), dim3(grid), dim3(256), 0, st, a);
+}
+
+// slabs per block that give `want` workgroups, at least `least`
+static int slabs_for(int nblk, int want, int least) {
+  int n = least;
+  while (n < NC && nblk * n < want) n <<= 1;
+  return n;
 }
 
 static void launch_stage(FusedState &f, const DevCfg &c, hipStream_t st, int stage) {
   FusedArgs a = make_args(f, c);
-  bool visc = c.visc_eta != 0.0;
+  const bool visc = c.visc_eta != 0.0;
+  if (c.nv == 5) a.nslab = slabs_for(f.nblk, HYDRO_WANT, 1);
   // z slabs: the delta-form MHD kernels without viscosity (the viscous
   // epilogue works one plane behind and needs whole columns)
-  if (!f.fp64 && c.nv == 8 && !f.mhd_plain32 && !visc) a.nslab = f.nslab;
+  else if (!f.fp64 && !f.mhd_plain32 && !visc) a.nslab = f.nslab > 0 ? f.nslab : 1;
   const int items = f.nblk * a.nslab;
-  int grid = f.grid > 0 ? std::min(f.grid, items) : items;
-  if (f.fp64) launch_stage_t<double, double>(a, grid, c.nv, c.pd.solver, visc, stage, 0, st);
-  else launch_stage_t<float, float>(a, grid, c.nv, c.pd.solver, visc, stage, f.mhd_plain32, st);
+  const int grid = f.grid > 0 ? std::min(f.grid, items) : items;
+  if (c.nv == 8) launch_stage_mhd(f, a, grid, c.pd.solver, visc, stage, st);
+  else if (f.fp64) launch_hydro<double, double>(a, grid, stage, st);
+  else launch_hydro<float, float>(a, grid, stage, st);
+}
+
+// what follows the second stage's kernel
+static void launch_rest(FusedState &f, const DevCfg &c, hipStream_t st) {
+  if (c.nv != 5) return;
+  FusedArgs a = make_args(f, c);
+  a.nslab = slabs_for(f.nblk, END_WANT, NC / END_PLANES);
+  if (f.fp64) launch_end<double, double>(a, st);
+  else launch_end<float, float>(a, st);
 }
 
 static void enqueue_step(FusedState &f, const DevCfg &c, hipStream_t st) {
-  hipLaunchKernelGGL(k_dt_finalize, dim3(1), dim3(1), 0, st, f.step, c.cfl, c.cooling);
+  hipLaunchKernelGGL(k_begin, dim3(1), dim3(64), 0, st, f.step, f.slots, c.cfl, c.cooling);
   launch_stage(f, c, st, 1);
   launch_stage(f, c, st, 2);
-  hipLaunchKernelGGL(k_step_post, dim3(1), dim3(1), 0, st, f.step);
+  launch_rest(f, c, st);
 }
 
 // after a step of the two-buffer form the new state is in the other buffer
@@ -316,6 +392,7 @@ int fused_run(FusedState &f, const DevCfg &c, hipStream_t st, int nsteps, int *i
   s.nextout = *nextout;
   s.dtout = dtout;
   s.t_sc = t_sc;
+  s.open = 0;
   FCHK(hipMemcpyAsync(f.step, &s, sizeof(s), hipMemcpyHostToDevice, st));
   hipGraphExec_t ex[2];
   if (step_graphs(f, c, st, ex)) return 1;
@@ -330,6 +407,7 @@ int fused_run(FusedState &f, const DevCfg &c, hipStream_t st, int nsteps, int *i
   float ms = 0;
   hipEventElapsedTime(&ms, f.ev[0], f.ev[1]);
   f.t_tot = nsteps > 0 ? ms / nsteps : 0.0;
+  step_close(&s);
   *it = s.it;
   *dt = s.dt;
   *time = s.time;
@@ -342,13 +420,13 @@ int fused_run(FusedState &f, const DevCfg &c, hipStream_t st, int nsteps, int *i
 int fused_time_stages(FusedState &f, const DevCfg &c, hipStream_t st, int reps) {
   float a1 = 0, a2 = 0;
   for (int r = 0; r < reps; r++) {
-    hipLaunchKernelGGL(k_dt_finalize, dim3(1), dim3(1), 0, st, f.step, c.cfl, c.cooling);
+    hipLaunchKernelGGL(k_begin, dim3(1), dim3(64), 0, st, f.step, f.slots, c.cfl, c.cooling);
     FCHK(hipEventRecord(f.ev[0], st));
     launch_stage(f, c, st, 1);
     FCHK(hipEventRecord(f.ev[1], st));
     launch_stage(f, c, st, 2);
+    launch_rest(f, c, st);
     FCHK(hipEventRecord(f.ev[2], st));
-    hipLaunchKernelGGL(k_step_post, dim3(1), dim3(1), 0, st, f.step);
     swap_u(f);
     FCHK(hipEventSynchronize(f.ev[2]));
     float m1, m2;

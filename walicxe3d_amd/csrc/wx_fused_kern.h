@@ -23,10 +23,12 @@ struct FusedArgs {
   double *Uout;      // stage 2 output (in place)
   const void *UPin;  // stage 2 input (storage type ST)
   void *UPout;       // stage 1 output
+  double *X;         // state the second stage leaves for k_end
+  unsigned long long *slots;   // partial minima of dt (DT_SLOTS)
   const int *order;
   StepState *step;
   int nblk;
-  int nslab;         // z slabs per block, one workgroup each (FP32 MHD kernels without viscosity; else 1)
+  int nslab;         // z slabs per block, one workgroup each
 };
 
 template <typename RF> __device__ __forceinline__ const Phys<RF> &phys(const DevCfg &c);

@@ -23,8 +23,7 @@ void plain_update(const DevCfg &c, const UserSource &us, const double *U, const 
 void plain_finish(const DevCfg &c, const double *UP, double *U, double *P, StepState *ss, double mu0,
                   unsigned long long *slots, hipStream_t st);
 // the step's scalars from the slots (P: reduced from it first)
-void plain_step_begin(const DevCfg &c, const double *P, StepState *ss, unsigned long long *slots, int advance,
-                      hipStream_t st);
+void plain_step_begin(const DevCfg &c, const double *P, StepState *ss, unsigned long long *slots, hipStream_t st);
 void plain_viscous(const DevCfg &c, const double *UP, double *U, hipStream_t st);
 void plain_timestep(const DevCfg &c, const double *P, unsigned long long *slots, unsigned long long *dtbits,
                     hipStream_t st);

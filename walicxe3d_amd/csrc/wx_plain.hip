@@ -657,28 +657,20 @@ __global__ void __launch_bounds__(256) k_finish(DevCfg c, const double *UP, doub
   if (slots) dt_to_slot(dtmin, blockIdx.x, slots);
 }
 
-// The scalars of a step: closes the step before it (advance), then dt from
-// the smallest of the slots with the start-up ramp and the output clamp
-// (source/hydro_solver.f90:183-207).  The slots are cleared for the next
-// reduction.  One wavefront.
-__global__ void __launch_bounds__(64) k_step_begin(StepState *s, unsigned long long *slots, double cfl, int cooling,
-                                                   int advance) {
-  static_assert(DT_SLOTS == 64, "one slot per lane");
-  double m = __longlong_as_double((long long)slots[threadIdx.x * DT_STRIDE]);
-  slots[threadIdx.x * DT_STRIDE] = ~0ull;
-  // an untouched slot reads as a NaN, which fmin drops
-  for (int off = 32; off > 0; off >>= 1) m = fmin(m, __shfl_xor(m, off));
+// The scalars of a step: closes the step before it, then dt from the smallest
+// of the slots with the start-up ramp and the output clamp
+// (source/hydro_solver.f90:183-207).  One wavefront.
+__global__ void __launch_bounds__(64) k_step_begin(StepState *s, unsigned long long *slots, double cfl, int cooling) {
+  const double m = fold_slots(slots);
   if (threadIdx.x == 0) {
-    if (advance) step_close(s);
+    step_close(s);
     step_open(s, m, cfl, cooling);
   }
 }
 
 // the smallest of the slots into *out, the slots cleared
 __global__ void __launch_bounds__(64) k_dt_fold(unsigned long long *slots, unsigned long long *out) {
-  double m = __longlong_as_double((long long)slots[threadIdx.x * DT_STRIDE]);
-  slots[threadIdx.x * DT_STRIDE] = ~0ull;
-  for (int off = 32; off > 0; off >>= 1) m = fmin(m, __shfl_xor(m, off));
+  const double m = fold_slots(slots);
   if (threadIdx.x == 0) *out = (unsigned long long)__double_as_longlong(m);
 }
 
@@ -916,10 +908,9 @@ void plain_timestep(const DevCfg &c, const double *P, unsigned long long *slots,
   launch_timestep(c, P, slots, st);
   hipLaunchKernelGGL(k_dt_fold, dim3(1), dim3(64), 0, st, slots, dtbits);
 }
-void plain_step_begin(const DevCfg &c, const double *P, StepState *ss, unsigned long long *slots, int advance,
-                      hipStream_t st) {
+void plain_step_begin(const DevCfg &c, const double *P, StepState *ss, unsigned long long *slots, hipStream_t st) {
   if (P) launch_timestep(c, P, slots, st);
-  hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(64), 0, st, ss, slots, c.cfl, c.cooling, advance);
+  hipLaunchKernelGGL(k_step_begin, dim3(1), dim3(64), 0, st, ss, slots, c.cfl, c.cooling);
 }
 void plain_cooling(const DevCfg &c, double *U, double *P, double dt, double mu0, hipStream_t st) {
   hipLaunchKernelGGL(k_cooling, dim3(16, c.nblk), dim3(256), 0, st, c, U, P, dt, mu0);
