@@ -18,7 +18,8 @@ struct FusedState {
   // into this second buffer, and the two swap roles every step
   double *U2 = nullptr;
   int two_u = 0;
-  // hydro: the state between the second stage and the end of the step
+  // the state between the second stage and the end of the step, where that is
+  // a kernel of its own (hydro, FP64, viscous FP32 MHD)
   double *X = nullptr;
   unsigned long long *slots = nullptr;   // partial minima of dt, next to step's dtmin_bits
   void *UP = nullptr;        // [blk][nv][4096] half-step state (FP32, or FP64 in the fp64 variant)

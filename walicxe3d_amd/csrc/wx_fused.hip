@@ -36,8 +36,10 @@ namespace wx {
 // for HYDRO_WANT = 512, 1024, 2048, 4096: 64 blocks 58.9, 56.1, 56.3, 55.5; 904
 // blocks on 4 levels 519, 478, 466, 472; 1728 blocks 759, 758, 749, 761.  The
 // end of the step runs 4 planes per workgroup, fewer below END_WANT: 64 blocks
-// 52.6, 56.1, 55.6 for 512, 1024, 2048.
-constexpr int HYDRO_WANT = 2048, END_WANT = 512;
+// 52.6, 56.1, 55.6 for 512, 1024, 2048.  FP32 MHD (two workgroups per CU) takes
+// slabs below MHD_WANT unless set_tuning chose: 64 blocks 87.7, 67.0, 76.9 for
+// 256, 512, 1024; 32 blocks 57.2, 47.5, 47.3; whole blocks took 265 and 270.
+constexpr int HYDRO_WANT = 2048, END_WANT = 512, MHD_WANT = 512;
 
 static thread_local std::string f_err;
 const char *fused_error() { return f_err.c_str(); }
@@ -155,7 +157,7 @@ int fused_alloc(FusedState &f, const DevCfg &c, const std::vector<BlockInfo> &in
   FCHK(hipMalloc(&f.UP, n * (f.fp64 ? sizeof(double) : sizeof(float))));
   FCHK(hipMalloc(&f.order, c.nblk * sizeof(int)));
   FCHK(hipMalloc(&f.step, sizeof(StepState)));
-  if (c.nv == 5) FCHK(hipMalloc(&f.X, n * sizeof(double)));
+  if (!f.two_u || ends_apart(c)) FCHK(hipMalloc(&f.X, n * sizeof(double)));
   FCHK(hipMalloc(&f.slots, DT_SLOTS * DT_STRIDE * sizeof(unsigned long long)));
   f.host_info = info;
   f.maxlev = c.maxlev;
@@ -263,48 +265,34 @@ int fused_timestep(FusedState &f, const DevCfg &c, hipStream_t st, double *dt_ra
   return 0;
 }
 
-// FP64 MHD stages, and the FP32 MHD forms
-static void launch_stage_mhd(const FusedState &f, const FusedArgs &a, int grid, int solver, bool visc, int stage,
-                             hipStream_t st) {
-  if (!f.fp64) launch_stage_mhd32(a, grid, solver, visc, stage, f.mhd_plain32, st);
-  else if (solver == SOLVER_HLLD) launch_stage_s<double, double, 8, SOLVER_HLLD>(a, grid, visc, stage, st);
-  else launch_stage_s<double, double, 8, SOLVER_HLLE>(a, grid, visc, stage, st);
-}
-
 // meshes without wind sources take kernels without the wind code; minmod, the
 // default limiter, is fixed at compile time, the others are read at run time
-template <typename RF, typename ST, int SOLVER, bool WINDS>
-static void launch_hydro_t(const FusedArgs &a, int grid, int stage, hipStream_t st) {
+template <int NV, typename RF, typename ST, int SOLVER, bool WINDS>
+static void launch_flow_t(const FusedArgs &a, int grid, int stage, hipStream_t st) {
   constexpr int MM = 1;   // LIMITER_MINMOD (source/constants.f90)
   if (stage == 1)
-    hipLaunchKernelGGL((k_hydro<false, RF, ST, SOLVER, MM, WINDS>), dim3(grid), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((k_flow<NV, false, RF, ST, SOLVER, MM, WINDS>), dim3(grid), dim3(256), 0, st, a);
   else if (a.c.pf.limiter == MM)
-    hipLaunchKernelGGL((k_hydro<true, RF, ST, SOLVER, MM, WINDS>), dim3(grid), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((k_flow<NV, true, RF, ST, SOLVER, MM, WINDS>), dim3(grid), dim3(256), 0, st, a);
   else
-    hipLaunchKernelGGL((k_hydro<true, RF, ST, SOLVER, LIM_RUNTIME, WINDS>), dim3(grid), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((k_flow<NV, true, RF, ST, SOLVER, LIM_RUNTIME, WINDS>), dim3(grid), dim3(256), 0, st, a);
 }
 
-template <typename RF, typename ST>
-static void launch_hydro(const FusedArgs &a, int grid, int stage, hipStream_t st) {
-  const bool winds = a.c.nwind > 0;
-  if (a.c.pd.solver == SOLVER_HLLC) {
-    if (winds) launch_hydro_t<RF, ST, SOLVER_HLLC, true>(a, grid, stage, st);
-    else launch_hydro_t<RF, ST, SOLVER_HLLC, false>(a, grid, stage, st);
-  } else {
-    if (winds) launch_hydro_t<RF, ST, SOLVER_HLL, true>(a, grid, stage, st);
-    else launch_hydro_t<RF, ST, SOLVER_HLL, false>(a, grid, stage, st);
-  }
+template <int NV, typename RF, typename ST, int SOLVER>
+static void launch_flow(const FusedArgs &a, int grid, int stage, hipStream_t st) {
+  if (a.c.nwind > 0) launch_flow_t<NV, RF, ST, SOLVER, true>(a, grid, stage, st);
+  else launch_flow_t<NV, RF, ST, SOLVER, false>(a, grid, stage, st);
 }
 
-template <typename RF, typename ST>
+template <int NV, typename RF, typename ST>
 static void launch_end(const FusedArgs &a, hipStream_t st) {
   const int grid = a.nblk * a.nslab;
   if (a.c.visc_eta == 0.0)
-    hipLaunchKernelGGL((k_end<5, RF, ST, false, false, false>), dim3(grid), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((k_end<NV, RF, ST, false, false, false>), dim3(grid), dim3(256), 0, st, a);
   else if (a.c.nwind > 0)
-    hipLaunchKernelGGL((k_end<5, RF, ST, true, false, true>), dim3(grid), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((k_end<NV, RF, ST, true, false, true>), dim3(grid), dim3(256), 0, st, a);
   else
-    hipLaunchKernelGGL((k_end<5, RF, ST, true, false, false>), dim3(grid), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((k_end<NV, RF, ST, true, false, false>), dim3(grid), dim3(256), 0, st, a);
 }
 
 // slabs per block that give `want` workgroups, at least `least`
@@ -316,25 +304,36 @@ static int slabs_for(int nblk, int want, int least) {
 
 static void launch_stage(FusedState &f, const DevCfg &c, hipStream_t st, int stage) {
   FusedArgs a = make_args(f, c);
-  const bool visc = c.visc_eta != 0.0;
-  if (c.nv == 5) a.nslab = slabs_for(f.nblk, HYDRO_WANT, 1);
-  // z slabs: the delta-form MHD kernels without viscosity (the viscous
-  // epilogue works one plane behind and needs whole columns)
-  else if (!f.fp64 && !f.mhd_plain32 && !visc) a.nslab = f.nslab > 0 ? f.nslab : 1;
+  const bool hllc = c.pd.solver == SOLVER_HLLC, hlld = c.pd.solver == SOLVER_HLLD;
+  const bool mhd32 = c.nv == 8 && !f.fp64;
+  if (!mhd32) a.nslab = slabs_for(f.nblk, HYDRO_WANT, 1);
+  else if (!f.mhd_plain32) a.nslab = f.nslab > 0 ? f.nslab : slabs_for(f.nblk, MHD_WANT, 1);
   const int items = f.nblk * a.nslab;
   const int grid = f.grid > 0 ? std::min(f.grid, items) : items;
-  if (c.nv == 8) launch_stage_mhd(f, a, grid, c.pd.solver, visc, stage, st);
-  else if (f.fp64) launch_hydro<double, double>(a, grid, stage, st);
-  else launch_hydro<float, float>(a, grid, stage, st);
+  if (mhd32) {
+    launch_stage_mhd32(a, grid, c.pd.solver, c.visc_eta != 0.0, stage, f.mhd_plain32, st);
+  } else if (c.nv == 8) {
+    if (hlld) launch_flow<8, double, double, SOLVER_HLLD>(a, grid, stage, st);
+    else launch_flow<8, double, double, SOLVER_HLLE>(a, grid, stage, st);
+  } else if (f.fp64) {
+    if (hllc) launch_flow<5, double, double, SOLVER_HLLC>(a, grid, stage, st);
+    else launch_flow<5, double, double, SOLVER_HLL>(a, grid, stage, st);
+  } else {
+    if (hllc) launch_flow<5, float, float, SOLVER_HLLC>(a, grid, stage, st);
+    else launch_flow<5, float, float, SOLVER_HLL>(a, grid, stage, st);
+  }
 }
 
-// what follows the second stage's kernel
+// the end of the step, where the second stage's kernel leaves it
 static void launch_rest(FusedState &f, const DevCfg &c, hipStream_t st) {
-  if (c.nv != 5) return;
+  const bool mhd32 = c.nv == 8 && !f.fp64;
+  if (mhd32 && (f.mhd_plain32 || !ends_apart(c))) return;
   FusedArgs a = make_args(f, c);
   a.nslab = slabs_for(f.nblk, END_WANT, NC / END_PLANES);
-  if (f.fp64) launch_end<double, double>(a, st);
-  else launch_end<float, float>(a, st);
+  if (mhd32) launch_end_mhd32(a, st);
+  else if (c.nv == 8) launch_end<8, double, double>(a, st);
+  else if (f.fp64) launch_end<5, double, double>(a, st);
+  else launch_end<5, float, float>(a, st);
 }
 
 static void enqueue_step(FusedState &f, const DevCfg &c, hipStream_t st) {
@@ -447,7 +446,7 @@ int fused_time_stages(FusedState &f, const DevCfg &c, hipStream_t st, int reps) 
 // kind 2: block order along the Morton (0) or the Hilbert (1) curve
 // kind 3: FP32 MHD fluxes in delta form (0) or plain FP32 (1)
 // kind 4: z slabs per block (1, 2, 4, 8), one workgroup each, in the
-//         delta-form MHD kernels without viscosity (no effect elsewhere)
+//         delta-form MHD kernels (by mesh size until set; no effect elsewhere)
 int fused_set_tuning(FusedState &f, int kind, int value) {
   if (kind < 0 || kind > 4) return 1;
   if ((kind == 2 || kind == 3) && (value < 0 || value > 1)) return 1;

@@ -18,8 +18,10 @@ void launch_stage_mhd32(const FusedArgs &a, int grid, int solver, bool visc, int
     else launch_stage_s<float, float, 8, SOLVER_HLLE>(a, grid, visc, stage, st);
     return;
   }
-  if (solver == SOLVER_HLLD) launch_mhd<SOLVER_HLLD>(a, grid, visc, stage, st);
-  else launch_mhd<SOLVER_HLLE>(a, grid, visc, stage, st);
+  if (solver == SOLVER_HLLD) launch_mhd<SOLVER_HLLD>(a, grid, stage, st);
+  else launch_mhd<SOLVER_HLLE>(a, grid, stage, st);
 }
+
+void launch_end_mhd32(const FusedArgs &a, hipStream_t st) { launch_mhd_end(a, st); }
 
 }  // namespace wx

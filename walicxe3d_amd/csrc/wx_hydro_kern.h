@@ -1,5 +1,5 @@
-// wx_hydro_kern.h - the stage kernels of the fused hydro form and the kernel
-// that ends a step.
+// wx_hydro_kern.h - the stage kernels of the fused hydro form and of FP64 MHD,
+// and the kernel that ends a step.
 //
 // One workgroup of 256 lanes updates L planes of a block; lane (i, j) owns a
 // column.  Per plane the primitives of the plane and its x/y face halo sit in
@@ -88,15 +88,20 @@ __device__ __forceinline__ void stage_prims(const Phys<double> &pd, const Phys<R
 }
 
 // rot for y where d holds, per lane
-template <typename R> __device__ __forceinline__ void rot_y_if(bool d, R *v) {
+template <int NV, typename R> __device__ __forceinline__ void rot_y_if(bool d, R *v) {
   const R a = v[1], b = v[2];
   v[1] = d ? b : a;
   v[2] = d ? a : b;
+  if constexpr (NV == 8) {
+    const R e = v[5], f = v[6];
+    v[5] = d ? f : e;
+    v[6] = d ? e : f;
+  }
 }
 
 // limited states and flux of one face in the x-aligned order
 template <int NV, int SOLVER, int LIM, bool S2, typename RF>
-__device__ __forceinline__ void hydro_face(const Phys<RF> &P, const RF *pll, RF *pl, RF *pr, const RF *prr, RF *ff) {
+__device__ __forceinline__ void flow_face(const Phys<RF> &P, const RF *pll, RF *pl, RF *pr, const RF *prr, RF *ff) {
   if constexpr (S2) {
     if constexpr (LIM == LIM_RUNTIME) {
       limit_all<NV>(pll, pl, pr, prr, P.limiter);
@@ -106,17 +111,20 @@ __device__ __forceinline__ void hydro_face(const Phys<RF> &P, const RF *pll, RF 
     }
   }
   if constexpr (SOLVER == SOLVER_HLLC) primfhllc_sel(P, pl, pr, ff);
+  else if constexpr (SOLVER == SOLVER_HLLD) primfhlld_sel(P, pl, pr, ff);
+  else if constexpr (SOLVER == SOLVER_HLLE) primfhlle(P, pl, pr, ff);
   else primfhll(P, pl, pr, ff);
 }
 
-template <bool S2, typename RF, typename ST, int SOLVER, int LIM, bool WINDS>
-__global__ void __launch_bounds__(256, sizeof(RF) == 4 ? 4 : 2) k_hydro(FusedArgs a) {
-  constexpr int NV = 5;
+template <int NV, bool S2, typename RF, typename ST, int SOLVER, int LIM, bool WINDS>
+__global__ void __launch_bounds__(256, sizeof(RF) == 4 ? 4 : 2) k_flow(FusedArgs a) {
+  constexpr bool MHD = NV == 8;
   constexpr int H = S2 ? 2 : 1;            // halo depth of the stencil
   constexpr int W = NC + 2 * H;
   constexpr int WP = W | 1;                // LDS row pitch
   constexpr int NX = NC + 1;
-  constexpr int NW = S2 ? 4 : 2;           // planes in the column window
+  constexpr int NW = S2 ? 4 : (MHD ? 3 : 2);   // planes in the column window
+  constexpr int C = NW - 1 - H;                // plane k in the window (with k-1 for the second order and Powell)
   using T = typename std::conditional<S2, ST, double>::type;
   __shared__ RF sp[NV][W * WP];            // primitives of the plane and its x/y halo
   __shared__ RF sfx[NV][NC * NX];          // x fluxes [v][(j-1)*17 + s]
@@ -126,6 +134,7 @@ __global__ void __launch_bounds__(256, sizeof(RF) == 4 ? 4 : 2) k_hydro(FusedArg
   Phys<RF> P = phys<RF>(c);
   Phys<double> pd = c.pd;
   P.nv = pd.nv = NV;
+  P.mhd = pd.mhd = MHD;
   const T *in;
   if constexpr (S2) in = static_cast<const ST *>(a.UPin);
   else in = a.U;
@@ -152,6 +161,9 @@ __global__ void __launch_bounds__(256, sizeof(RF) == 4 ? 4 : 2) k_hydro(FusedArg
     const int k0 = slab * L + 1, k1 = k0 + L - 1;
     const int l = c.info[b].level - 1;
     const double dtdx = dtp / c.dx[0][l], dtdy = dtp / c.dx[1][l], dtdz = dtp / c.dx[2][l];
+    // (RF)(1.0 / (2.0 * dx)): central differences of Powell's source
+    const RF idx2 = (RF)(1.0 / (2.0 * c.dx[0][l])), idy2 = (RF)(1.0 / (2.0 * c.dx[1][l])),
+             idz2 = (RF)(1.0 / (2.0 * c.dx[2][l]));
     RF win[NW][NV], fzp[NV];
     // Iteration k loads plane k + H of the column; the first iterations only
     // fill the window (one call site of the load, with its ghost paths).
@@ -176,8 +188,8 @@ __global__ void __launch_bounds__(256, sizeof(RF) == 4 ? 4 : 2) k_hydro(FusedArg
         RF pll[NV], pl[NV], pr[NV], prr[NV];
 #pragma unroll
         for (int v = 0; v < NV; v++) {
-          pl[v] = win[S2 ? 1 : 0][v];
-          pr[v] = win[S2 ? 2 : 1][v];
+          pl[v] = win[C][v];
+          pr[v] = win[C + 1][v];
           if constexpr (S2) {
             pll[v] = win[0][v];
             prr[v] = win[NW - 1][v];
@@ -189,13 +201,13 @@ __global__ void __launch_bounds__(256, sizeof(RF) == 4 ? 4 : 2) k_hydro(FusedArg
           rot<NV>(2, pll);
           rot<NV>(2, prr);
         }
-        hydro_face<NV, SOLVER, LIM, S2>(P, pll, pl, pr, prr, fzc);
+        flow_face<NV, SOLVER, LIM, S2>(P, pll, pl, pr, prr, fzc);
         rot<NV>(2, fzc);
       }
       if (k >= k0) {
         // the faces of the plane below were solved before the last barrier
 #pragma unroll
-        for (int v = 0; v < NV; v++) sp[v][own] = win[S2 ? 1 : 0][v];
+        for (int v = 0; v < NV; v++) sp[v][own] = win[C][v];
         if (hth) {
           RF ph[NV];
           stage_prims<NV, RF, S2>(pd, P, uh, ph);
@@ -217,7 +229,7 @@ __global__ void __launch_bounds__(256, sizeof(RF) == 4 ? 4 : 2) k_hydro(FusedArg
               prr[v] = x[2];
             }
           }
-          hydro_face<NV, SOLVER, LIM, S2>(P, pll, pl, pr, prr, ff);
+          flow_face<NV, SOLVER, LIM, S2>(P, pll, pl, pr, prr, ff);
 #pragma unroll
           for (int v = 0; v < NV; v++) sfx[v][tj * NX + ti] = ff[v];
         }
@@ -241,10 +253,17 @@ __global__ void __launch_bounds__(256, sizeof(RF) == 4 ? 4 : 2) k_hydro(FusedArg
             rot<NV>(1, pll);
             rot<NV>(1, prr);
           }
-          hydro_face<NV, SOLVER, LIM, S2>(P, pll, pl, pr, prr, ff);
+          flow_face<NV, SOLVER, LIM, S2>(P, pll, pl, pr, prr, ff);
           rot<NV>(1, ff);
 #pragma unroll
           for (int v = 0; v < NV; v++) sfy[v][tj * NC + ti] = ff[v];
+        }
+        // Powell's div B of the plane, while its primitives are in LDS
+        RF divB = RF(0);
+        if constexpr (MHD) {
+          if (c.eight_wave)
+            divB = (sp[5][own + 1] - sp[5][own - 1]) * idx2 + (sp[6][own + WP] - sp[6][own - WP]) * idy2 +
+                   (win[C + 1][7] - win[C - 1][7]) * idz2;
         }
         // the 16 x and 16 y faces s = 16 on the last 32 lanes
         if (tid >= 256 - 2 * NC) {
@@ -262,14 +281,14 @@ __global__ void __launch_bounds__(256, sizeof(RF) == 4 ? 4 : 2) k_hydro(FusedArg
               prr[v] = x[2 * st];
             }
           }
-          rot_y_if(d, pl);
-          rot_y_if(d, pr);
+          rot_y_if<NV>(d, pl);
+          rot_y_if<NV>(d, pr);
           if constexpr (S2) {
-            rot_y_if(d, pll);
-            rot_y_if(d, prr);
+            rot_y_if<NV>(d, pll);
+            rot_y_if<NV>(d, prr);
           }
-          hydro_face<NV, SOLVER, LIM, S2>(P, pll, pl, pr, prr, ff);
-          rot_y_if(d, ff);
+          flow_face<NV, SOLVER, LIM, S2>(P, pll, pl, pr, prr, ff);
+          rot_y_if<NV>(d, ff);
 #pragma unroll
           for (int v = 0; v < NV; v++) *(d ? &sfy[v][NC * NC + aa] : &sfx[v][aa * NX + NC]) = ff[v];
         }
@@ -286,13 +305,29 @@ __global__ void __launch_bounds__(256, sizeof(RF) == 4 ? 4 : 2) k_hydro(FusedArg
 #pragma unroll
             for (int v = 0; v < NV; v++) ub[v] = ws[v];
         }
+        double un[NV];
+#pragma unroll
+        for (int v = 0; v < NV; v++)
+          un[v] = ub[v] + dtdx * ((double)sfx[v][tj * NX + ti] - (double)sfx[v][tj * NX + ti + 1]) +
+                  dtdy * ((double)sfy[v][tj * NC + ti] - (double)sfy[v][(tj + 1) * NC + ti]) +
+                  dtdz * ((double)fzp[v] - (double)fzc[v]);
+        if constexpr (MHD) {
+          if (c.eight_wave) {
+            // Powell source (source/sources.f90:38-95) from the stage primitives
+            const RF *pp = win[C];
+            un[1] += dtp * (double)(-divB * pp[5]);
+            un[2] += dtp * (double)(-divB * pp[6]);
+            un[3] += dtp * (double)(-divB * pp[7]);
+            un[4] += dtp * (double)(-divB * (pp[1] * pp[5] + pp[2] * pp[6] + pp[3] * pp[7]));
+            un[5] += dtp * (double)(-divB * pp[1]);
+            un[6] += dtp * (double)(-divB * pp[2]);
+            un[7] += dtp * (double)(-divB * pp[3]);
+          }
+        }
 #pragma unroll
         for (int v = 0; v < NV; v++) {
-          const double un = ub[v] + dtdx * ((double)sfx[v][tj * NX + ti] - (double)sfx[v][tj * NX + ti + 1]) +
-                            dtdy * ((double)sfy[v][tj * NC + ti] - (double)sfy[v][(tj + 1) * NC + ti]) +
-                            dtdz * ((double)fzp[v] - (double)fzc[v]);
-          if constexpr (S2) a.X[at + v * NINT] = un;
-          else static_cast<ST *>(a.UPout)[at + v * NINT] = (ST)un;
+          if constexpr (S2) a.X[at + v * NINT] = un[v];
+          else static_cast<ST *>(a.UPout)[at + v * NINT] = (ST)un[v];
         }
       }
 #pragma unroll
@@ -311,8 +346,12 @@ __global__ void __launch_bounds__(256, sizeof(RF) == 4 ? 4 : 2) k_hydro(FusedArg
 // ---------------------------------------------------------------------------
 constexpr int END_PLANES = 4;   // most planes per workgroup
 
+// whether the delta-form MHD kernels leave the end of the step to k_end: with
+// viscosity (neighbours) or cooling (its FP64 code, even unexecuted, spills)
+inline bool ends_apart(const DevCfg &c) { return c.visc_eta != 0.0 || c.cooling; }
+
 template <int NV, typename RF, typename ST, bool VISC, bool DEL, bool WINDS>
-__global__ void __launch_bounds__(256, 3) k_end(FusedArgs a) {
+__global__ void __launch_bounds__(256, NV == 8 ? 2 : 3) k_end(FusedArgs a) {
   __shared__ RF ring[VISC ? NV : 1][END_PLANES * 4 * NC];   // [v][plane][side][position]
   __shared__ double sred[4];
   const DevCfg &c = a.c;

@@ -18,10 +18,19 @@
 // Stage 1 writes the half-step state as FP32 increments over U^n; stage 2
 // reads U^n of neighbour blocks for its halo and so writes U^{n+1} into the
 // second state buffer (the two swap roles every step).
+//
+// Bound: latency and VALU issue at the 2 waves per SIMD that 256 VGPRs and
+// 62 KB of LDS leave.  With viscosity or cooling the second stage leaves its
+// state to k_end (TO_X): inside, that code held one workgroup per CU (82 KB of
+// LDS) and spilled.  8 viscous HLLE blocks, whole blocks -> 16 slabs: first
+// stage 81 -> 10 us, second 275 -> 23 + 9 us; 64 HLLD blocks, 8 slabs: 105 ->
+// 24 and 145 -> 36 us; 4096 blocks: 1.04 and 1.55 -> 1.51 ms (without the FP64
+// cooling code the second stage keeps its 18 VGPRs out of scratch).
 #pragma once
 
 #include "wx_delta.h"
 #include "wx_fused_kern.h"
+#include "wx_hydro_kern.h"
 
 namespace wx {
 
@@ -109,19 +118,17 @@ __device__ __forceinline__ void face_flux(const DevCfg &c, double *wl, double *w
 #define WX_MHD_MIN_WAVES 2
 #endif
 
-template <bool S2, bool VISC, int SOLVER, int LIM, bool WIND>
+template <bool S2, bool TO_X, int SOLVER, int LIM, bool WIND>
 __global__ void __launch_bounds__(256, WX_MHD_MIN_WAVES) k_mhd(FusedArgs a) {
   constexpr int NV = 8;
   constexpr int H = S2 ? 2 : 1;            // halo depth of the stencil
   constexpr int W = NC + 2 * H;
   constexpr int WPD = W | 1;               // LDS row pitch (FP64 elements)
   constexpr int NW = S2 ? 4 : 3;           // planes in the column window
-  constexpr bool SV = S2 && VISC;
   constexpr int NXF = (NC + 1) * NC;       // x (or y) faces of a plane
   __shared__ double sw[NV][W * WPD];       // FP64 primitives of plane k (cross region)
   __shared__ double sfx[NV][NXF];          // x fluxes [v][row * 17 + s]
   __shared__ double sfy[NV][NXF];          // y fluxes [v][col * 17 + s]
-  __shared__ float sun[SV ? 2 : 1][SV ? NV : 1][NC + 2][NC + 2];  // UP_new planes + half-step ghost ring
   __shared__ double sred[4];
 
   const DevCfg &c = a.c;
@@ -159,16 +166,17 @@ __global__ void __launch_bounds__(256, WX_MHD_MIN_WAVES) k_mhd(FusedArgs a) {
     else { hj = side ? NC + g : 1 - g; hi = aa; }
   };
 
-  // Work items: block bi of the order list, z slab s of it (planes
-  // s L + 1 .. (s + 1) L, L = NC / nslab; the viscous kernels run whole
-  // blocks, nslab = 1).  A slab starts one plane early, at its bottom z face,
-  // which the slab below computes too, with the same code and inputs.
+  // Work items: block bi of the order list, z slab of it (planes slab L + 1 ..
+  // (slab + 1) L, L = NC / nslab).  A slab starts one plane early, at its
+  // bottom z face, which the slab below computes too, with the same code and
+  // inputs.
   const int nslab = uni(a.nslab);
-  WX_EMU_CHECK(nslab >= 1 && NC % nslab == 0 && (!SV || nslab == 1));
+  WX_EMU_CHECK(nslab >= 1 && NC % nslab == 0);
   const int L = NC / nslab;
   for (int item = blockIdx.x; item < a.nblk * nslab; item += gridDim.x) {
-    const int bi = item / nslab;
-    const int k0 = (item - bi * nslab) * L + 1, k1 = k0 + L - 1;
+    int bi, slab;
+    item_of(item, a.nblk, nslab, bi, slab);
+    const int k0 = slab * L + 1, k1 = k0 + L - 1;
     // block, level and per-block constants are the same in every lane:
     // scalar registers
     const int b = uni(a.order[bi]);
@@ -182,9 +190,7 @@ __global__ void __launch_bounds__(256, WX_MHD_MIN_WAVES) k_mhd(FusedArgs a) {
     // S2: planes {k-1, k, k+1, k+2};  S1: planes {k-1, k, k+1}
     double wq[NW][NV];
     double ucol[NV];
-    double ughost_lo[SV ? NV : 1], ughost_hi[SV ? NV : 1];   // half-step ghosts at planes 0 and 17
-    double fzp[NV];                                          // z flux (k-1 | k)
-    double unew_prev[SV ? NV : 1], unew_prev2[SV ? NV : 1];  // UP_new at planes k-1, k-2 (viscosity)
+    double fzp[NV];                        // z flux (k-1 | k)
 #pragma unroll
     for (int w = 0; w < NW; w++)
 #pragma unroll
@@ -214,14 +220,6 @@ __global__ void __launch_bounds__(256, WX_MHD_MIN_WAVES) k_mhd(FusedArgs a) {
         const int kn = S2 ? k + 2 : k + 1;
         if constexpr (S2) load_cell<float, NV, true, true, WIND>(a, UPin, b, i, j, kn, ucol);
         else load_cell<double, NV, false, false, WIND>(a, a.U, b, i, j, kn, ucol);
-        if constexpr (SV) {
-          if (kn == 0)
-#pragma unroll
-            for (int v = 0; v < NV; v++) ughost_lo[v] = ucol[v];
-          if (kn == NC + 1)
-#pragma unroll
-            for (int v = 0; v < NV; v++) ughost_hi[v] = ucol[v];
-        }
         prims64(icv, ucol, wq[NW - 1]);
       }
       if constexpr (LW) {
@@ -232,7 +230,6 @@ __global__ void __launch_bounds__(256, WX_MHD_MIN_WAVES) k_mhd(FusedArgs a) {
           for (int v = 0; v < NV; v++) sw[v][own] = wq[1][v];
       }
       double wh[NV];                       // halo cell primitives
-      float uhf[SV ? NV : 1];              // halo cell state (viscosity ring)
       auto halo_load = [&]() {
         int hi, hj, hg;
         halo_cell(hi, hj, hg);
@@ -240,10 +237,6 @@ __global__ void __launch_bounds__(256, WX_MHD_MIN_WAVES) k_mhd(FusedArgs a) {
         if constexpr (S2) load_cell<float, NV, true, true, WIND>(a, UPin, b, hi, hj, k, uh);
         else load_cell<double, NV, false, false, WIND>(a, a.U, b, hi, hj, k, uh);
         prims64(icv, uh, wh);
-        if constexpr (SV) {
-#pragma unroll
-          for (int v = 0; v < NV; v++) uhf[v] = (float)uh[v];
-        }
       };
       if (EARLY_HALO && hth && k >= k0) halo_load();
       if (k < k0 - 1) continue;
@@ -273,11 +266,6 @@ __global__ void __launch_bounds__(256, WX_MHD_MIN_WAVES) k_mhd(FusedArgs a) {
         halo_cell(hi, hj, hg);
 #pragma unroll
         for (int v = 0; v < NV; v++) sw[v][(hj - 1 + H) * WPD + (hi - 1 + H)] = wh[v];
-        if constexpr (SV) {
-          if (hg == 1)
-#pragma unroll
-            for (int v = 0; v < NV; v++) sun[k & 1][v][hj][hi] = uhf[v];
-        }
       }
       __syncthreads();
       // x faces s = 0..15 of plane k, one per lane (row tj, face ti)
@@ -389,46 +377,18 @@ __global__ void __launch_bounds__(256, WX_MHD_MIN_WAVES) k_mhd(FusedArgs a) {
       for (int v = 0; v < NV; v++) fzp[v] = fzc[v];
       if constexpr (!S2) continue;
 
-      // ---- stage 2 epilogue: viscosity (one plane behind), prims, dt
-      if constexpr (SV) {
+      // stage 2: the state for k_end, or the end of the step here
+      if constexpr (TO_X) {
+        double *Xo = a.X + (size_t)b * NV * NINT + lin(i, j, k);
 #pragma unroll
-        for (int v = 0; v < NV; v++) sun[k & 1][v][j][i] = (float)unew[v];
-        __syncthreads();
-        if (k > 1) {
-          const int pb = (k - 1) & 1;
-          double ufin[NV];
-#pragma unroll
-          for (int v = 0; v < NV; v++) {
-            double below = (k - 2 == 0) ? ughost_lo[v] : unew_prev2[v];
-            double lap = (double)sun[pb][v][j][i + 1] + (double)sun[pb][v][j][i - 1] +
-                         (double)sun[pb][v][j + 1][i] + (double)sun[pb][v][j - 1][i] + below + unew[v] -
-                         6.0 * unew_prev[v];
-            ufin[v] = unew_prev[v] + c.visc_eta * lap;
-          }
-          finish_cell<NV, float>(a, b, i, j, k - 1, dt, ufin, dxl, dyl, dzl, dtmin);
-        }
-#pragma unroll
-        for (int v = 0; v < NV; v++) { unew_prev2[v] = unew_prev[v]; unew_prev[v] = unew[v]; }
+        for (int v = 0; v < NV; v++) Xo[v * NINT] = unew[v];
       } else {
-        finish_cell<NV, float>(a, b, i, j, k, dt, unew, dxl, dyl, dzl, dtmin);
+        finish_cell32<NV, false>(a, b, i, j, k, unew, dxl, dyl, dzl, dtmin);
       }
-    }
-    if constexpr (SV) {
-      // plane 16: its upper neighbour is the half-step ghost at plane 17
-      __syncthreads();
-      const int pb = NC & 1;
-      double ufin[NV];
-#pragma unroll
-      for (int v = 0; v < NV; v++) {
-        double lap = (double)sun[pb][v][j][i + 1] + (double)sun[pb][v][j][i - 1] + (double)sun[pb][v][j + 1][i] +
-                     (double)sun[pb][v][j - 1][i] + unew_prev2[v] + ughost_hi[v] - 6.0 * unew_prev[v];
-        ufin[v] = unew_prev[v] + c.visc_eta * lap;
-      }
-      finish_cell<NV, float>(a, b, i, j, NC, dt, ufin, dxl, dyl, dzl, dtmin);
     }
     __syncthreads();
   }
-  if constexpr (S2) {
+  if constexpr (S2 && !TO_X) {
     // exact min: wavefront shuffles, then one 64-bit atomic per workgroup on
     // the bit pattern (positive doubles order like their bits)
     for (int off = 32; off > 0; off >>= 1) dtmin = fmin(dtmin, __shfl_xor(dtmin, off));
@@ -436,31 +396,43 @@ __global__ void __launch_bounds__(256, WX_MHD_MIN_WAVES) k_mhd(FusedArgs a) {
     __syncthreads();
     if (tid == 0) {
       double m = fmin(fmin(sred[0], sred[1]), fmin(sred[2], sred[3]));
-      atomicMin(&a.step->dtmin_bits, (unsigned long long)__double_as_longlong(m));
+      atomicMin(&a.slots[(blockIdx.x % DT_SLOTS) * DT_STRIDE], (unsigned long long)__double_as_longlong(m));
     }
   }
 }
 
+// with viscosity or cooling the second stage leaves its state to k_end (to_x)
 template <int SOLVER, bool WIND>
-inline void launch_mhd_w(const FusedArgs &a, int grid, bool visc, int stage, hipStream_t st) {
+inline void launch_mhd_w(const FusedArgs &a, int grid, bool to_x, int stage, hipStream_t st) {
   constexpr int MM = 1;  // LIMITER_MINMOD (source/constants.f90)
   const bool mm = a.c.pf.limiter == MM && !WIND;
   if (stage == 1)
     hipLaunchKernelGGL((k_mhd<false, false, SOLVER, LIM_RUNTIME, WIND>), dim3(grid), dim3(256), 0, st, a);
-  else if (visc)
-    hipLaunchKernelGGL((k_mhd<true, true, SOLVER, LIM_RUNTIME, WIND>), dim3(grid), dim3(256), 0, st, a);
+  else if (to_x)   // one instance for meshes with and without sources
+    hipLaunchKernelGGL((k_mhd<true, true, SOLVER, LIM_RUNTIME, true>), dim3(grid), dim3(256), 0, st, a);
   else if (mm)
     hipLaunchKernelGGL((k_mhd<true, false, SOLVER, MM, false>), dim3(grid), dim3(256), 0, st, a);
   else
     hipLaunchKernelGGL((k_mhd<true, false, SOLVER, LIM_RUNTIME, WIND>), dim3(grid), dim3(256), 0, st, a);
 }
 
+inline void launch_mhd_end(const FusedArgs &a, hipStream_t st) {
+  const int grid = a.nblk * a.nslab;
+  if (a.c.visc_eta == 0.0)
+    hipLaunchKernelGGL((k_end<8, float, float, false, true, false>), dim3(grid), dim3(256), 0, st, a);
+  else if (a.c.nwind > 0)
+    hipLaunchKernelGGL((k_end<8, float, float, true, true, true>), dim3(grid), dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL((k_end<8, float, float, true, true, false>), dim3(grid), dim3(256), 0, st, a);
+}
+
 // meshes with wind sources take the kernels that carry the wind code (every
 // limiter at run time); the others leave it out
 template <int SOLVER>
-inline void launch_mhd(const FusedArgs &a, int grid, bool visc, int stage, hipStream_t st) {
-  if (a.c.nwind > 0) launch_mhd_w<SOLVER, true>(a, grid, visc, stage, st);
-  else launch_mhd_w<SOLVER, false>(a, grid, visc, stage, st);
+inline void launch_mhd(const FusedArgs &a, int grid, int stage, hipStream_t st) {
+  const bool to_x = ends_apart(a.c);
+  if (a.c.nwind > 0) launch_mhd_w<SOLVER, true>(a, grid, to_x, stage, st);
+  else launch_mhd_w<SOLVER, false>(a, grid, to_x, stage, st);
 }
 
 }  // namespace wx
