@@ -198,6 +198,72 @@ __device__ __forceinline__ void load_cell(const FusedArgs &a, const T *W, int b,
   }
 }
 
+// Where a lane's ghosts of a block lie, found once per block and kept in LDS
+// (the kernels have no registers to spare): ghost_source reduced to what does
+// not change along a lane's column.  Asking it in every plane put its table
+// reads, and the data reads that depend on them, between two barriers.
+// blk < 0: left to load_cell (averages over finer cells; without WALLS also
+// reflective faces: the negation cost the FP32 hydro kernels 3 %, 1728 blocks
+// 0.705 against 0.681 ms a step).
+//
+// The column of source cells of one x/y ghost column: plane k of the source
+// (same level, domain faces) or plane (k + 1) / 2 of the half of it that the
+// block touches (coarser).
+struct HaloRef {
+  int blk, where;   // cell in its plane (8 bits), coarser (1), first plane of the half (4), variable negated from bit 16
+  __device__ __forceinline__ int at(int k) const {
+    const int half = (where >> 8) & 1, kk = ((k + half) >> half) + ((where >> 9) & 15);
+    WX_EMU_CHECK(kk >= 1 && kk <= NC);
+    return (kk - 1) * NC * NC + (where & 255);
+  }
+  __device__ __forceinline__ int flip() const { return where >> 16; }
+};
+
+// The face records are read as scalars and selected by lane (b uniform)
+template <bool WALLS>
+__device__ __forceinline__ HaloRef halo_ref(const FusedArgs &a, int b, int hi, int hj) {
+  const BlockInfo &B = a.c.info[b];
+  const bool xs = hi < 1 || hi > NC;                   // an x face, else a y face
+  const bool low = xs ? hi < 1 : hj < 1;
+  const int g = xs ? (low ? 1 - hi : hi - NC) : (low ? 1 - hj : hj - NC);
+  const int aa = xs ? hj : hi;
+  auto pick = [&](int l, int r, int f, int k) { return xs ? (low ? l : r) : (low ? f : k); };
+  const int type = pick(B.face[LEFT].type, B.face[RIGHT].type, B.face[FRONT].type, B.face[BACK].type);
+  const int src = pick(B.face[LEFT].src[0], B.face[RIGHT].src[0], B.face[FRONT].src[0], B.face[BACK].src[0]);
+  const int bc = pick(a.c.bc[LEFT], a.c.bc[RIGHT], a.c.bc[FRONT], a.c.bc[BACK]);
+  int blk = src, cn, ca = aa, half = 0, flip = 0;
+  if (type == NEIGH_SAME) cn = low ? NC + 1 - g : g;
+  else if (type == NEIGH_COARSER) {
+    half = 1;
+    cn = low ? NC : 1;
+    ca = (aa + 1) / 2 + (xs ? B.sib[1] : B.sib[0]) * (NC / 2);
+  } else if (type == NEIGH_FINER) return HaloRef{-1, 0};
+  else {   // domain boundary
+    blk = b;
+    const bool wall = bc == BC_REFLECTIVE;
+    cn = low ? (wall ? g : 1) : NC + 1 - g;
+    if (!WALLS && wall) return HaloRef{-1, 0};
+    flip = wall ? (xs ? 1 : 2) : 0;
+  }
+  const int i = xs ? cn : ca, j = xs ? ca : cn;
+  return HaloRef{blk, ((j - 1) * NC + i - 1) | (half << 8) | ((half ? B.sib[2] * (NC / 2) : 0) << 9) | (flip << 16)};
+}
+
+// The two ghosts of a lane's z-column below (f BOTTOM) or above (TOP) a block
+struct ColRef {
+  int blk, where;   // cells of layers 1 and 2 in the source (12 bits each, the second from bit 16), bit 12: 3 negated
+  __device__ __forceinline__ int at(int g) const { return (g == 1 ? where : where >> 16) & 0xfff; }
+  __device__ __forceinline__ int flip() const { return (where >> 12) & 1 ? 3 : 0; }
+};
+
+__device__ __forceinline__ ColRef col_ref(const FusedArgs &a, int b, int f, int i, int j) {
+  GhostSrc s, t;
+  ghost_source(a.c.info, a.c.bc, b, f, 1, i, j, s);
+  ghost_source(a.c.info, a.c.bc, b, f, 2, i, j, t);
+  if (s.kind == 1) return ColRef{-1, 0};
+  return ColRef{s.blk, lin(s.c[0], s.c[1], s.c[2]) | (lin(t.c[0], t.c[1], t.c[2]) << 16) | ((s.kind == 2) << 12)};
+}
+
 // MHD primitives for the FP32 kernels (flow2prim, source/hydro_core.f90:
 // 323-378, with its floors): one reciprocal of the density for the
 // velocities; the pressure from the FP64 state in FP64 when fp64 (the

@@ -129,6 +129,11 @@ __global__ void __launch_bounds__(256, sizeof(RF) == 4 ? 4 : 2) k_flow(FusedArgs
   __shared__ RF sp[NV][W * WP];            // primitives of the plane and its x/y halo
   __shared__ RF sfx[NV][NC * NX];          // x fluxes [v][(j-1)*17 + s]
   __shared__ RF sfy[NV][NX * NC];          // y fluxes [v][s*16 + (i-1)]
+  // sources of the halo found once per block (1728 blocks 0.749 -> 0.683 ms a
+  // step, 904 on four levels 466 -> 449 us); not with wind code (over 30 VGPRs
+  // pushed out: 500 -> 536 us) nor in FP64 (343 -> 349 us)
+  constexpr bool HREF = !WINDS && sizeof(RF) == 4;
+  __shared__ HaloRef sref[HREF ? 4 * H * NC : 1];
 
   const DevCfg &c = a.c;
   Phys<RF> P = phys<RF>(c);
@@ -164,6 +169,7 @@ __global__ void __launch_bounds__(256, sizeof(RF) == 4 ? 4 : 2) k_flow(FusedArgs
     // (RF)(1.0 / (2.0 * dx)): central differences of Powell's source
     const RF idx2 = (RF)(1.0 / (2.0 * c.dx[0][l])), idy2 = (RF)(1.0 / (2.0 * c.dx[1][l])),
              idz2 = (RF)(1.0 / (2.0 * c.dx[2][l]));
+    if (HREF && hth) sref[tid] = halo_ref<false>(a, b, hi, hj);   // read back by the lane that wrote it
     RF win[NW][NV], fzp[NV];
     // Iteration k loads plane k + H of the column; the first iterations only
     // fill the window (one call site of the load, with its ghost paths).
@@ -181,7 +187,16 @@ __global__ void __launch_bounds__(256, sizeof(RF) == 4 ? 4 : 2) k_flow(FusedArgs
       }
       if (k < k0 - 1) continue;
       T uh[NV];
-      if (hth && k >= k0) load_state<T, NV, S2, WINDS>(a, in, b, hi, hj, k, uh);
+      if (hth && k >= k0) {
+        const HaloRef href = HREF ? sref[tid] : HaloRef{-1, 0};
+        if (href.blk >= 0) {
+          const T *S = in + (size_t)href.blk * NV * NINT + href.at(k);
+#pragma unroll
+          for (int v = 0; v < NV; v++) uh[v] = S[v * NINT];
+        } else {
+          load_state<T, NV, S2, WINDS>(a, in, b, hi, hj, k, uh);
+        }
+      }
       // z flux (k | k+1)
       RF fzc[NV];
       {

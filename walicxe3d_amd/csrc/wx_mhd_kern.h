@@ -19,13 +19,17 @@
 // reads U^n of neighbour blocks for its halo and so writes U^{n+1} into the
 // second state buffer (the two swap roles every step).
 //
-// Bound: latency and VALU issue at the 2 waves per SIMD that 256 VGPRs and
-// 62 KB of LDS leave.  With viscosity or cooling the second stage leaves its
-// state to k_end (TO_X): inside, that code held one workgroup per CU (82 KB of
-// LDS) and spilled.  8 viscous HLLE blocks, whole blocks -> 16 slabs: first
-// stage 81 -> 10 us, second 275 -> 23 + 9 us; 64 HLLD blocks, 8 slabs: 105 ->
-// 24 and 145 -> 36 us; 4096 blocks: 1.04 and 1.55 -> 1.51 ms (without the FP64
-// cooling code the second stage keeps its 18 VGPRs out of scratch).
+// Bound: VALU issue and latency at the 2 waves per SIMD that 256 VGPRs and
+// 67 KB of LDS leave.  The x/y halo used to ask for its source cell in every
+// plane, between two barriers; now the sources are found once per block
+// (HaloRef, ColRef), the loads of the next plane are issued before the last
+// barrier of this one, two barriers a plane remain of three, the waves take
+// turns with the 32 outer faces, and the window fills in one go: 4096 HLLD
+// blocks 2.54 -> 2.23 ms a step, HLLE 2.21 -> 1.98 ms, 64 HLLD blocks 66.5 -> 65.5 us.
+// With viscosity or cooling the second stage leaves its state to k_end (TO_X):
+// inside, that code held one workgroup per CU (82 KB of LDS) and spilled.
+// 8 viscous HLLE blocks, whole blocks -> 16 slabs: first stage 81 -> 10 us,
+// second 275 -> 23 + 9 us.
 #pragma once
 
 #include "wx_delta.h"
@@ -130,6 +134,8 @@ __global__ void __launch_bounds__(256, WX_MHD_MIN_WAVES) k_mhd(FusedArgs a) {
   __shared__ double sfx[NV][NXF];          // x fluxes [v][row * 17 + s]
   __shared__ double sfy[NV][NXF];          // y fluxes [v][col * 17 + s]
   __shared__ double sred[4];
+  __shared__ HaloRef sref[4 * H * NC];     // sources of the x/y halo of lanes tid < 4 H 16
+  __shared__ ColRef scol[2][256];          // and of the column's ghosts; each read back by its lane
 
   const DevCfg &c = a.c;
   const Phys<float> &P = c.pf;
@@ -144,16 +150,17 @@ __global__ void __launch_bounds__(256, WX_MHD_MIN_WAVES) k_mhd(FusedArgs a) {
   double dtmin = 1.0e30;
 
   // x/y face halo of a plane, H layers on each of the 4 sides: lanes
-  // tid < NH load one cell each.  The first stage issues these loads at the
-  // top of the plane (their latency overlaps the z face); the second, whose
-  // registers are full there, after the first barrier.
+  // tid < NH load one cell each.
   constexpr int NH = 4 * H * NC;
-  constexpr bool EARLY_HALO = !S2;
   // second stage: plane k of the column window lives in this lane's slot of
   // sw (where the x/y faces read it) rather than in registers, from the
   // point where it is stored until it is read back as plane k-1
   constexpr bool LW = S2;
   const int own = (j - 1 + H) * WPD + (i - 1 + H);
+  // Loads one plane ahead, except where they push over 40 VGPRs out: with wind
+  // code (8 viscous blocks 54.1 against 51.7 us a step) and in the HLLE second
+  // stage (64 blocks 60 against 57.7 us, though 4096 blocks 1.94 against 1.98 ms)
+  constexpr bool PIPE = !WIND && !(S2 && SOLVER == SOLVER_HLLE);
   const bool hth = tid < NH;
   // halo cell (hi, hj) of lane tid, layer g
   auto halo_cell = [&](int &hi, int &hj, int &g) {
@@ -186,21 +193,150 @@ __global__ void __launch_bounds__(256, WX_MHD_MIN_WAVES) k_mhd(FusedArgs a) {
     const double dtdx = uni(dtp / dxl), dtdy = uni(dtp / dyl), dtdz = uni(dtp / dzl);
     const double idx2 = uni(1.0 / (2.0 * dxl)), idy2 = uni(1.0 / (2.0 * dyl)), idz2 = uni(1.0 / (2.0 * dzl));
 
+    const bool winds = WIND && a.c.nwind > 0;
+    if (k0 - H < 1) scol[0][tid] = col_ref(a, b, BOTTOM, i, j);
+    if (k1 + H > NC) scol[1][tid] = col_ref(a, b, TOP, i, j);
+    if (hth) {
+      int hi, hj, hg;
+      halo_cell(hi, hj, hg);
+      sref[tid] = halo_ref<true>(a, b, hi, hj);
+    }
+    // element 0 of the column's cell in plane kn; false: that takes load_cell
+    auto col_at = [&](int kn, size_t &at) -> bool {
+      WX_EMU_CHECK(kn >= k0 - H && kn <= k1 + H);
+      if (winds) return false;
+      const bool own = kn >= 1 && kn <= NC;
+      int blk = b, cell = 0;
+      if (own) cell = lin(i, j, kn);
+      else {
+        const ColRef r = scol[kn < 1 ? 0 : 1][tid];
+        blk = uni(r.blk);
+        cell = r.at(kn < 1 ? 1 - kn : kn - NC);
+      }
+      at = (size_t)blk * NV * NINT + cell;
+      return blk >= 0;
+    };
     // column window of FP64 primitives: at iteration k (after the shift)
     // S2: planes {k-1, k, k+1, k+2};  S1: planes {k-1, k, k+1}
     double wq[NW][NV];
-    double ucol[NV];
     double fzp[NV];                        // z flux (k-1 | k)
 #pragma unroll
     for (int w = 0; w < NW; w++)
 #pragma unroll
       for (int v = 0; v < NV; v++) wq[w][v] = 0.0;
 
-    // Iteration k loads plane k + NW - 2 into the window.  The first
-    // iterations only fill it (S2: planes k0-2 .. k0, S1: plane k0-1), so
-    // that one call site of load_cell, with its ghost paths, serves every
-    // plane: the kernel's code stays small.
-    for (int k = k0 - (S2 ? 4 : 2); k <= k1; k++) {
+    // (a reflective face negates the normal momentum, where the value is used)
+    auto col_flip = [&](int kn, double *u) {
+      if (kn >= 1 && kn <= NC) return;
+      if (!winds && scol[kn < 1 ? 0 : 1][tid].flip()) u[3] = -u[3];
+    };
+
+    // Loads of iteration kl: plane kl + NW - 2 of the column and plane kl of
+    // the halo, with PIPE issued while iteration kl - 1 works.  In the second stage the
+    // FP32 increments wait beside the state and are added where it is used
+    // (-0 where the state is whole: it leaves every bit of a sum).
+    double ucol[NV], uh[NV];
+    float dcol[NV], dh[NV];
+#pragma unroll
+    for (int v = 0; v < NV; v++) { ucol[v] = uh[v] = 1.0; dcol[v] = dh[v] = -0.0f; }
+    auto fetch = [&](int kl) {
+      // (nothing of the consumed values stays alive)
+#pragma unroll
+      for (int v = 0; v < NV; v++) { ucol[v] = uh[v] = 1.0; dcol[v] = dh[v] = -0.0f; }
+      if (kl > k1) return;
+      const int kn = S2 ? kl + 2 : kl + 1;
+      size_t at;
+      if (col_at(kn, at)) {
+#pragma unroll
+        for (int v = 0; v < NV; v++) ucol[v] = a.U[at + v * NINT];
+        if constexpr (S2)
+#pragma unroll
+          for (int v = 0; v < NV; v++) dcol[v] = UPin[at + v * NINT];
+      } else {
+        if constexpr (S2) load_cell<float, NV, true, true, WIND>(a, UPin, b, i, j, kn, ucol);
+        else load_cell<double, NV, false, false, WIND>(a, a.U, b, i, j, kn, ucol);
+        if constexpr (S2)
+#pragma unroll
+          for (int v = 0; v < NV; v++) dcol[v] = -0.0f;
+      }
+      if (hth && kl >= k0) {
+        int hi, hj, hg;
+        halo_cell(hi, hj, hg);
+        const HaloRef href = sref[tid];
+        if (href.blk >= 0) {
+          const size_t at = (size_t)href.blk * NV * NINT + href.at(kl);
+#pragma unroll
+          for (int v = 0; v < NV; v++) uh[v] = a.U[at + v * NINT];
+          if constexpr (S2)
+#pragma unroll
+            for (int v = 0; v < NV; v++) dh[v] = UPin[at + v * NINT];
+        } else {
+          if constexpr (S2) load_cell<float, NV, true, true, false>(a, UPin, b, hi, hj, kl, uh);
+          else load_cell<double, NV, false, false, false>(a, a.U, b, hi, hj, kl, uh);
+          if constexpr (S2)
+#pragma unroll
+            for (int v = 0; v < NV; v++) dh[v] = -0.0f;
+        }
+        if constexpr (WIND) {
+          double w[MAXV];
+          if (a.c.nwind > 0 && wind_state(a.c, b, hi, hj, kl, w)) {
+#pragma unroll
+            for (int v = 0; v < NV; v++) uh[v] = w[v];
+            if (href.flip() == 1) uh[1] = -uh[1];   // negated again where it is used
+            if (href.flip() == 2) uh[2] = -uh[2];
+            if constexpr (S2)
+#pragma unroll
+              for (int v = 0; v < NV; v++) dh[v] = -0.0f;
+          }
+        }
+      }
+    };
+
+    // The window's first planes (S2: k0-2 .. k0 and the loads of k0+1; S1:
+    // k0-1 and the loads of k0) all at once, if none of them needs load_cell;
+    // otherwise the first iterations fill it, one plane each (with PIPE the
+    // very first only issues loads), so that one call site of load_cell serves
+    // every plane: the kernel's code stays small.
+    constexpr int BACK0 = (S2 ? 4 : 2) + PIPE;
+    int kf = k0 - BACK0;
+    {
+      size_t at[S2 ? 4 : 2];
+      bool all = true;
+#pragma unroll
+      for (int w = 0; w < (S2 ? 4 : 2); w++) all = col_at(k0 - H + w, at[w]) && all;
+      if (all) {
+        constexpr int NF = S2 ? 3 : 1;
+        double uf[NF][NV];
+        float df[NF][NV];
+#pragma unroll
+        for (int w = 0; w < NF; w++)
+#pragma unroll
+          for (int v = 0; v < NV; v++) {
+            uf[w][v] = a.U[at[w] + v * NINT];
+            if constexpr (S2) df[w][v] = UPin[at[w] + v * NINT];
+          }
+        if constexpr (PIPE)
+#pragma unroll
+          for (int v = 0; v < NV; v++) {
+            ucol[v] = a.U[at[NF] + v * NINT];
+            if constexpr (S2) dcol[v] = UPin[at[NF] + v * NINT];
+          }
+#pragma unroll
+        for (int w = 0; w < NF; w++) {
+          if constexpr (S2)
+#pragma unroll
+            for (int v = 0; v < NV; v++) uf[w][v] = uf[w][v] + (double)df[w][v];
+          col_flip(k0 - H + w, uf[w]);
+          prims64(icv, uf[w], wq[NW - NF + w]);
+        }
+        if constexpr (LW)
+#pragma unroll
+          for (int v = 0; v < NV; v++) sw[v][own] = wq[1][v];
+        kf = k0 - 1;
+      }
+    }
+    for (int k = kf; k <= k1; k++) {
+      if constexpr (!PIPE) fetch(k);
       if constexpr (LW) {
         // plane k-1 from this lane's slot of the plane store, where the
         // previous iteration left it
@@ -216,33 +352,32 @@ __global__ void __launch_bounds__(256, WX_MHD_MIN_WAVES) k_mhd(FusedArgs a) {
 #pragma unroll
           for (int v = 0; v < NV; v++) wq[w][v] = wq[w + 1][v];
       }
-      {
-        const int kn = S2 ? k + 2 : k + 1;
-        if constexpr (S2) load_cell<float, NV, true, true, WIND>(a, UPin, b, i, j, kn, ucol);
-        else load_cell<double, NV, false, false, WIND>(a, a.U, b, i, j, kn, ucol);
-        prims64(icv, ucol, wq[NW - 1]);
-      }
-      if constexpr (LW) {
-        // while the window fills, the slot takes plane k here (later after
-        // the first barrier, with the rest of the plane)
-        if (k < k0)
+      if constexpr (S2)
 #pragma unroll
-          for (int v = 0; v < NV; v++) sw[v][own] = wq[1][v];
-      }
-      double wh[NV];                       // halo cell primitives
-      auto halo_load = [&]() {
+        for (int v = 0; v < NV; v++) ucol[v] = ucol[v] + (double)dcol[v];
+      if (!PIPE || k > k0 - BACK0) col_flip(k + NW - 2, ucol);
+      prims64(icv, ucol, wq[NW - 1]);
+      // own primitives of plane k and, by the halo lanes, its face halo into
+      // LDS: the previous plane's readers were done at the last barrier
+      if (LW || k >= k0)
+#pragma unroll
+        for (int v = 0; v < NV; v++) sw[v][own] = wq[1][v];
+      if (hth && k >= k0) {
         int hi, hj, hg;
         halo_cell(hi, hj, hg);
-        double uh[NV];
-        if constexpr (S2) load_cell<float, NV, true, true, WIND>(a, UPin, b, hi, hj, k, uh);
-        else load_cell<double, NV, false, false, WIND>(a, a.U, b, hi, hj, k, uh);
+        double wh[NV];
+        if constexpr (S2)
+#pragma unroll
+          for (int v = 0; v < NV; v++) uh[v] = uh[v] + (double)dh[v];
+        if (sref[tid].flip() == 1) uh[1] = -uh[1];
+        if (sref[tid].flip() == 2) uh[2] = -uh[2];
         prims64(icv, uh, wh);
-      };
-      if (EARLY_HALO && hth && k >= k0) halo_load();
-      if (k < k0 - 1) continue;
+#pragma unroll
+        for (int v = 0; v < NV; v++) sw[v][(hj - 1 + H) * WPD + (hi - 1 + H)] = wh[v];
+      }
       // z flux (k | k+1): one code path for every plane, the bottom face included
       double fzc[NV];
-      {
+      if (k >= k0 - 1) {
         double wl[NV], wr[NV];
 #pragma unroll
         for (int v = 0; v < NV; v++) {
@@ -251,21 +386,11 @@ __global__ void __launch_bounds__(256, WX_MHD_MIN_WAVES) k_mhd(FusedArgs a) {
         }
         face_flux<2, SOLVER>(c, wl, wr, fzc);
       }
-      if (k == k0 - 1) {
+      if (k < k0) {
 #pragma unroll
         for (int v = 0; v < NV; v++) fzp[v] = fzc[v];
+        if constexpr (PIPE) fetch(k + 1);
         continue;
-      }
-      __syncthreads();   // the previous plane's LDS readers are done
-      // own primitives of plane k into LDS; halo threads add the face halo
-#pragma unroll
-      for (int v = 0; v < NV; v++) sw[v][own] = wq[1][v];
-      if (hth) {
-        if (!EARLY_HALO) halo_load();
-        int hi, hj, hg;
-        halo_cell(hi, hj, hg);
-#pragma unroll
-        for (int v = 0; v < NV; v++) sw[v][(hj - 1 + H) * WPD + (hi - 1 + H)] = wh[v];
       }
       __syncthreads();
       // x faces s = 0..15 of plane k, one per lane (row tj, face ti)
@@ -298,11 +423,12 @@ __global__ void __launch_bounds__(256, WX_MHD_MIN_WAVES) k_mhd(FusedArgs a) {
 #pragma unroll
         for (int v = 0; v < NV; v++) sfy[v][col * (NC + 1) + sy] = ff[v];
       }
-      // the 16 x and the 16 y faces s = 16 together on the last 32 lanes (x
+      // the 16 x and the 16 y faces s = 16 together on 32 lanes of one wave (x
       // on the first 16, y on the others): one solve per lane, the states
-      // rotated by lane (selects) into the x-aligned order of face_flux<0>
-      if (tid >= 256 - 2 * NC) {
-        const int e = tid - (256 - 2 * NC);
+      // rotated by lane (selects) into the x-aligned order of face_flux<0>.
+      // The waves take turns, plane by plane: they sit on different SIMDs.
+      const int e = tid - 64 * (k & 3);
+      if ((unsigned)e < 2 * NC) {
         const bool d = e >= NC;                                // y face
         const int aa = d ? e - NC : e;                         // row or column
         const int st = d ? WPD : 1;
@@ -321,14 +447,19 @@ __global__ void __launch_bounds__(256, WX_MHD_MIN_WAVES) k_mhd(FusedArgs a) {
 #pragma unroll
         for (int v = 0; v < NV; v++) (d ? sfy[v] : sfx[v])[aa * (NC + 1) + NC] = ff[v];
       }
+      const double *Ub = a.U + (size_t)b * NV * NINT + lin(i, j, k);
+      double ub[NV];
+#pragma unroll
+      for (int v = 0; v < NV; v++) ub[v] = Ub[v * NINT];
+      double divB = 0.0;
+      if (c.eight_wave)
+        divB = (sw[5][own + 1] - sw[5][own - 1]) * idx2 + (sw[6][own + WPD] - sw[6][own - WPD]) * idy2 +
+               (wq[2][7] - wq[0][7]) * idz2;
+      if constexpr (PIPE) fetch(k + 1);
       __syncthreads();
       // conservative update of cell (i, j, k) in FP64
       double unew[NV];
       {
-        const double *Ub = a.U + (size_t)b * NV * NINT + lin(i, j, k);
-        double ub[NV];
-#pragma unroll
-        for (int v = 0; v < NV; v++) ub[v] = Ub[v * NINT];
         // base of the update: U^n, or the wind state in a cell that a source
         // covers (each stage's boundary() imposes the sources through
         // userBoundary: source/godunov.f90:79,141, source/boundary.f90:61)
@@ -348,14 +479,11 @@ __global__ void __launch_bounds__(256, WX_MHD_MIN_WAVES) k_mhd(FusedArgs a) {
                     dtdz * (fzp[v] - fzc[v]);
         if (c.eight_wave) {
           // Powell source (source/sources.f90:38-95) from the stage primitives
-          const int q = own;
-          const double divB = (sw[5][q + 1] - sw[5][q - 1]) * idx2 + (sw[6][q + WPD] - sw[6][q - WPD]) * idy2 +
-                              (wq[2][7] - wq[0][7]) * idz2;
           double ppl[NV];
           const double *pp = wq[1];
           if constexpr (LW) {
 #pragma unroll
-            for (int v = 0; v < NV; v++) ppl[v] = sw[v][q];
+            for (int v = 0; v < NV; v++) ppl[v] = sw[v][own];
             pp = ppl;
           }
           unew[1] += dtp * (-divB * pp[5]);
