@@ -297,7 +297,7 @@ def main():
     dom_ms, dom_bytes, dom = (s2, b_stage2, "stage2") if s2 >= s1 else (s1, b_stage1, "stage1")
     achieved = dom_bytes / (dom_ms * 1e-3)
     kname = ("k_mhd<%s>" % ("S2" if dom == "stage2" else "S1")) if nv == 8 else \
-        ("k_stage<%d,%s>" % (nv, "S2" if dom == "stage2" else "S1"))
+        ("k_flow<%d,%s>" % (nv, "S2" if dom == "stage2" else "S1"))
     roof = {"bound": "hbm", "kernel": kname,
             "achieved": achieved / 1e9, "peak": HBM_PEAK / 1e9, "unit": "GB/s", "frac": achieved / HBM_PEAK,
             "traffic": traffic_from_profiles(w.name), "algorithmic_bytes_per_launch": dom_bytes,

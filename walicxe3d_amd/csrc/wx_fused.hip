@@ -1,22 +1,26 @@
 // wx_fused.hip - the fused FP32 form of the Godunov update.
 //
 // One stage = one kernel launch over all blocks of all levels.  A workgroup
-// of 256 threads owns a block; thread (ti, tj) owns the column (i, j) and
-// marches in k.  Per k-plane the primitives of the plane and its x/y face
-// halo sit in LDS (x and y fluxes), the column's primitives of the planes
-// around k sit in registers (z fluxes, Powell term).  Face halos are read
-// straight from the neighbour blocks' interiors with the AMR exchange rules
-// of wx_device.h - no ghost cells are stored in HBM.
+// of 256 threads owns a block, or a z slab of one on meshes of few blocks;
+// thread (ti, tj) owns the column (i, j) and marches in k.  Per k-plane the
+// primitives of the plane and its x/y face halo sit in LDS (x and y fluxes),
+// the column's primitives of the planes around k sit in registers (z fluxes,
+// Powell term).  Face halos are read straight from the neighbour blocks'
+// interiors with the AMR exchange rules of wx_device.h - no ghost cells are
+// stored in HBM.
 //
 // Precision: bulk flux/reconstruction arithmetic in FP32; conserved state U
 // and its accumulation U + dt*dF in FP64; stage-1 pressure recovery from the
-// FP64 state in FP64; the stage-2 epilogue (viscosity, primitives, cooling,
+// FP64 state in FP64; the end of the step (viscosity, primitives, cooling,
 // dt candidate) in FP64 on U^{n+1}; dt reduced as an exact min.
 //
 // Stage 1 (first order, dt/2): U^n (FP64) -> UP (FP32).
-// Stage 2 (second order, dt): UP, U^n -> U^{n+1} (in place), with the
-// artificial viscosity (its face neighbours are the half-step ghosts, as in
-// the reference), updatePrims, cooling and the next dt fused in.
+// Stage 2 (second order, dt): UP, U^n -> U^{n+1}, with the next dt.  With
+// artificial viscosity or cooling stage 2 leaves its state to k_end, which
+// applies both (the viscosity's face neighbours are the half-step ghosts, as
+// in the reference) and forms the next dt.
+// k_flow (hydro, FP64 MHD; wx_hydro_kern.h), k_mhd (FP32 MHD;
+// wx_mhd_kern.h), k_stage (MHD with plain FP32 fluxes, set_tuning kind 3).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

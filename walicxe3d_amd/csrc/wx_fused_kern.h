@@ -443,20 +443,19 @@ __global__ void __launch_bounds__(256, (NV == 8 && !S2) ? WX_MHD_STAGE1_MIN_WAVE
   constexpr int ORD = S2 ? 2 : 1;
   constexpr int H = ORD;
   constexpr int W = NC + 2 * H;
-  // LDS row pitch: odd (bank spread of y-direction reads); in the FP32 MHD
-  // second stage without viscosity 49, which is 17 mod 32, so a half-wave's
-  // x-face reads (rows of 17 interfaces) fall in distinct banks
-  constexpr int WP = (NV == 8 && S2 && !VISC && sizeof(RF) == 4) ? 49 : (W | 1);
+  // LDS row pitch: odd (bank spread of y-direction reads); in the second stage
+  // without viscosity 49, which is 17 mod 32, so a half-wave's x-face reads
+  // (rows of 17 interfaces) fall in distinct banks
+  constexpr int WP = (S2 && !VISC) ? 49 : (W | 1);
   constexpr int NW = S2 ? 4 : 3;               // planes in the column window
   constexpr bool SV = S2 && VISC;
   constexpr int NXF = (NC + 1) * NC;           // x (or y) interfaces per plane
   __shared__ RF sp[NV][W * WP];                 // primitives of the plane (cross region)
   __shared__ RF sfx[NV][NC * (NC + 1)];        // x fluxes [v][(j-1)*17 + s]
-  __shared__ RF sfy[NV][(NC + 1) * NC];        // y fluxes, see YT
-  // y-flux layout: YT (MHD kernels) stores [v][(i-1)*17 + s] like sfx, so the
-  // stores of consecutive lanes (consecutive s) and the update's reads (lanes
-  // along i, row pitch 17) hit distinct LDS banks; otherwise [v][s*16 + (i-1)]
-  constexpr bool YT = NV == 8;
+  // y fluxes [v][(i-1)*17 + s] like sfx: the stores of consecutive lanes
+  // (consecutive s) and the update's reads (lanes along i, row pitch 17) hit
+  // distinct LDS banks
+  __shared__ RF sfy[NV][(NC + 1) * NC];
   __shared__ RF sun[SV ? 2 : 1][SV ? NV : 1][NC + 2][NC + 2];  // UP_new planes + half-step ghost ring
   __shared__ double sred[4];
 
@@ -467,25 +466,21 @@ __global__ void __launch_bounds__(256, (NV == 8 && !S2) ? WX_MHD_STAGE1_MIN_WAVE
   const int tid = threadIdx.x;
   const int ti = tid & 15, tj = tid >> 4;
   const int i = ti + 1, j = tj + 1;
-  const double dt = NV == 8 ? uni(a.step->dt) : a.step->dt;
+  const double dt = uni(a.step->dt);
   const double dtp = S2 ? dt : dt / 2.0;
   double dtmin = 1.0e30;
 
   for (int bi = blockIdx.x; bi < a.nblk; bi += gridDim.x) {
     // the block and its level are the same in every lane (and every lane is
-    // active here, at the top of the block loop): in the MHD kernels they are
-    // read into scalar registers, so that block addresses and per-level
-    // values stay scalar
-    const int b = NV == 8 ? uni(a.order[bi]) : a.order[bi];
+    // active here, at the top of the block loop): read into scalar registers,
+    // so that block addresses and per-level values stay scalar
+    const int b = uni(a.order[bi]);
     WX_EMU_CHECK(b >= 0 && b < a.nblk);
-    const int l = NV == 8 ? uni(c.info[b].level - 1) : c.info[b].level - 1;
+    const int l = uni(c.info[b].level - 1);
     const double dxl = c.dx[0][l], dyl = c.dx[1][l], dzl = c.dx[2][l];
-    double dtdx = dtp / dxl, dtdy = dtp / dyl, dtdz = dtp / dzl;
-    RF idx2 = (RF)(1.0 / (2.0 * dxl)), idy2 = (RF)(1.0 / (2.0 * dyl)), idz2 = (RF)(1.0 / (2.0 * dzl));
-    if constexpr (NV == 8) {
-      dtdx = uni(dtdx); dtdy = uni(dtdy); dtdz = uni(dtdz);
-      idx2 = uni(idx2); idy2 = uni(idy2); idz2 = uni(idz2);
-    }
+    const double dtdx = uni(dtp / dxl), dtdy = uni(dtp / dyl), dtdz = uni(dtp / dzl);
+    const RF idx2 = uni((RF)(1.0 / (2.0 * dxl))), idy2 = uni((RF)(1.0 / (2.0 * dyl))),
+             idz2 = uni((RF)(1.0 / (2.0 * dzl)));
 
     // column window of primitives; at iteration k (after the shift)
     // S2: win = planes {k-1, k, k+1, k+2};  S1: win = {k-1, k, k+1}
@@ -607,7 +602,7 @@ __global__ void __launch_bounds__(256, (NV == 8 && !S2) ? WX_MHD_STAGE1_MIN_WAVE
           for (int v = 0; v < NV; v++) sfx[v][aa * (NC + 1) + s] = ff[v];
         } else {
 #pragma unroll
-          for (int v = 0; v < NV; v++) sfy[v][YT ? aa * (NC + 1) + s : s * NC + aa] = ff[v];
+          for (int v = 0; v < NV; v++) sfy[v][aa * (NC + 1) + s] = ff[v];
         }
       }
       __syncthreads();
@@ -629,10 +624,9 @@ __global__ void __launch_bounds__(256, (NV == 8 && !S2) ? WX_MHD_STAGE1_MIN_WAVE
 #pragma unroll
         for (int v = 0; v < NV; v++)
           unew[v] = ub[v] + dtdx * ((double)sfx[v][tj * (NC + 1) + ti] - (double)sfx[v][tj * (NC + 1) + ti + 1]) +
-                    dtdy * ((double)sfy[v][YT ? ti * (NC + 1) + tj : tj * NC + ti] -
-                            (double)sfy[v][YT ? ti * (NC + 1) + tj + 1 : (tj + 1) * NC + ti]) +
+                    dtdy * ((double)sfy[v][ti * (NC + 1) + tj] - (double)sfy[v][ti * (NC + 1) + tj + 1]) +
                     dtdz * ((double)fzp[v] - (double)fzc[v]);
-        if (NV == 8 && c.eight_wave) {
+        if (c.eight_wave) {
           // Powell source (source/sources.f90:38-95) from the stage primitives
           const int q = (j - 1 + H) * WP + (i - 1 + H);
           RF divB = (sp[5][q + 1] - sp[5][q - 1]) * idx2 + (sp[6][q + WP] - sp[6][q - WP]) * idy2 +

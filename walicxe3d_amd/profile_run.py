@@ -188,7 +188,7 @@ def _summarize(args):
              "write_scale = %.4f" % wscale]
     out = {}
     for k in fetch:
-        # the second-stage flag: first template argument of k_mhd, second of k_stage
+        # the second-stage flag: first template argument of k_mhd, second of k_flow and k_stage
         st = _stage_of(k)
         if st is None:
             continue
@@ -227,7 +227,7 @@ def _header(args, title):
 
 def _stage_of(k):
     """'stage1' / 'stage2' for a fused stage kernel name, else None."""
-    if "k_stage" not in k and "k_mhd" not in k:
+    if not any(n in k for n in ("k_stage<", "k_flow<", "k_mhd<")):
         return None
     targs = k.split("<", 1)[1].split(",")
     return "stage2" if "true" in targs[0 if "k_mhd" in k else 1] else "stage1"
