@@ -37,12 +37,12 @@ namespace wx {
 
 // Workgroups below which the hydro kernels take thinner slabs (a slab of L
 // planes solves L + 1 z faces and loads L + 3 planes per column).  us per step
-// for HYDRO_WANT = 512, 1024, 2048, 4096: 64 blocks 58.9, 56.1, 56.3, 55.5; 904
-// blocks on 4 levels 519, 478, 466, 472; 1728 blocks 759, 758, 749, 761.  The
+// for HYDRO_WANT = 512, 1024, 2048, 4096: 64 blocks 51.2, 49.9, 50.5, 50.4; 904
+// blocks on 4 levels 470, 424, 411, 423; 1728 blocks 618, 619, 615, 637.  The
 // end of the step runs 4 planes per workgroup, fewer below END_WANT: 64 blocks
-// 52.6, 56.1, 55.6 for 512, 1024, 2048.  FP32 MHD (two workgroups per CU) takes
-// slabs below MHD_WANT unless set_tuning chose: 64 blocks 87.7, 67.0, 76.9 for
-// 256, 512, 1024; 32 blocks 57.2, 47.5, 47.3; whole blocks took 265 and 270.
+// 51.0, 50.5, 52.6 for 256, 512, 1024.  FP32 MHD (two workgroups per CU) takes
+// slabs below MHD_WANT unless set_tuning chose: 64 blocks 83.4, 65.7, 76.3 for
+// 256, 512, 1024; 32 blocks 56.2, 47.3, 46.9; whole blocks took 265 and 270.
 constexpr int HYDRO_WANT = 2048, END_WANT = 512, MHD_WANT = 512;
 
 static thread_local std::string f_err;
