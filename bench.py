@@ -159,7 +159,7 @@ def main():
     # ---- fused FP32 form ----------------------------------------------------
     f = hip.Walicxe3D(w, form=hip.FUSED_FP32, bids=bids)
     f.upload(U0)
-    best = {"grid": 0, "xcd_map": 0, "curve": 0, "nslab": 1}
+    best = {"grid": 0, "xcd_map": 0, "curve": 0, "nslab": 0}
     if args.no_tune:
         f.set_tuning(0, best["grid"])
         f.set_tuning(1, best["xcd_map"])

@@ -310,9 +310,9 @@ int wx_write_vtk(void *ctx, const char *datadir, int noutput, int npassive, int 
    curve, kind 3 = the FP32 MHD kernels' fluxes in delta form (0: FP64
    physical flux plus FP32 Riemann correction, the default) or entirely in
    FP32 (1: faster, with FP32 rounding of every flux term), kind 4 = z slabs
-   per block (1, 2, 4 or 8), one workgroup each, in the delta-form MHD
-   kernels (more workgroups for meshes of few blocks; results unchanged; until
-   set, and in the hydro and FP64 kernels always, chosen by the mesh size). */
+   per block (1, 2, 4, 8 or 16), one workgroup each, in the delta-form MHD
+   kernels (more workgroups for meshes of few blocks; results unchanged), or 0,
+   the default and always in the hydro and FP64 kernels: by the mesh size. */
 int wx_set_tuning(void *ctx, int kind, int value);
 /* Advances `reps` more iterations launching each stage kernel on its own
    between HIP events on the library's stream (fused form; no reference

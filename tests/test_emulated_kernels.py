@@ -175,6 +175,26 @@ def test_z_slabs_leave_the_state_unchanged(emu, tmp_path):
             assert np.array_equal(o, outs[0]), w.name
 
 
+def test_slab_count_of_the_rule_can_be_set_and_given_back(emu, tmp_path):
+    """Kind 4 takes every count the rule by mesh size can choose (16 on these
+    8 blocks, viscous and inviscid) and 0 for the rule itself: the same state
+    bit for bit; other values stay refused."""
+    import dataclasses
+    for visc in (2.0e-3, 0.0):
+        w = dataclasses.replace(W.get("mhd_hlle"), visc_eta=visc)
+        outs = []
+        for nslab in ("0", "16", "1"):
+            p = str(tmp_path / ("rule_%g_%s.bin" % (visc, nslab)))
+            _write_input(p, w, hip.FUSED_FP32)
+            _run(emu, [p, "1"], str(tmp_path), EMU_NSLAB=nslab)
+            outs.append(np.fromfile(p + ".out"))
+        assert np.array_equal(outs[0], outs[1]) and np.array_equal(outs[0], outs[2]), visc
+    for nslab in ("3", "32", "-1"):
+        r = subprocess.run([emu, p, "1"], capture_output=True, text=True, cwd=str(tmp_path),
+                           env=dict(os.environ, ASAN_OPTIONS="detect_leaks=0", EMU_NSLAB=nslab))
+        assert r.returncode == 1 and "unknown tuning option" in r.stdout, nslab
+
+
 def test_emulation_reproduces_fused_fp64(emu, tmp_path, oracle):
     w = W.get("ot64")
     p = str(tmp_path / "ot64.bin")

@@ -7,9 +7,9 @@ fused stage kernels leave open:
   - block order: along the Morton or the Hilbert curve, as one range or as
     8 ranges mapped to XCDs (workgroup w runs on XCD w % 8, so each XCD's L2
     serves its own halo reads);
-  - sub-block tiling: each 16^3 block split into 1, 2, 4 or 8 z slabs, one
-    workgroup each (FP32 MHD kernels without viscosity), so that a mesh of
-    few blocks still fills the 256 CUs.
+  - sub-block tiling of the FP32 MHD kernels: z slabs per block, one
+    workgroup each, by the mesh size (the library's own rule) or a fixed
+    count.  Every other kernel takes its slabs by the mesh size.
 Each candidate runs a few timed steps (HIP events inside wx_run) on the live
 state; the state advances, so tune on a scratch context.
 """
@@ -22,8 +22,8 @@ NUM_CUS = 256
 
 
 def slab_choices(solver):
-    """z slabs per block the solver's kernels can use: the FP32 MHD form
-    without viscosity splits blocks; every other kernel runs whole blocks."""
+    """Fixed z-slab counts worth a measurement beside the library's rule: in
+    the FP32 MHD form 1, 2, 4 and 8, with viscosity whole blocks only."""
     from walicxe3d_amd import hip
     w = solver.w
     if solver.form != hip.FUSED_FP32 or w.nv != 8 or w.visc_eta != 0.0:
@@ -31,10 +31,21 @@ def slab_choices(solver):
     return (1, 2, 4, 8)
 
 
+def slab_counts(solver):
+    """What tune() tries: 0, slabs by the mesh size, always; fixed counts
+    only where the kernels take them (FP32 MHD)."""
+    from walicxe3d_amd import hip
+    if solver.form != hip.FUSED_FP32 or solver.w.nv != 8:
+        return (0,)
+    return (0,) + slab_choices(solver)
+
+
 def candidates(nblk, slabs=(1,)):
+    """(grid, xcd_map, curve, nslab) to try; nslab 0: by the mesh size, whose
+    work items are at least the blocks."""
     out = []
     for nslab in slabs:
-        items = nblk * nslab
+        items = nblk * max(nslab, 1)
         grids = [0] + [k * NUM_CUS for k in (2, 4, 8) if k * NUM_CUS < items]
         out += [(g, x, c, nslab) for g, x, c in itertools.product(grids, (1, 0), (0, 1))]
     return out
@@ -47,9 +58,9 @@ def tune(solver, steps=3, verbose=False):
     """Try every candidate on `solver` (a hip.Walicxe3D in a fused form),
     then the CONFIRM fastest again with 4x the steps; returns (best, table)
     with best = {"grid": g, "xcd_map": x, "curve": c (0 Morton, 1 Hilbert),
-    "nslab": s, "ms": t, "ms_confirm": t2}, chosen by ms_confirm."""
+    "nslab": s (0 by the mesh size), "ms": t, "ms_confirm": t2}, chosen by ms_confirm."""
     table = []
-    for grid, xcd, curve, nslab in candidates(solver.nblk, slab_choices(solver)):
+    for grid, xcd, curve, nslab in candidates(solver.nblk, slab_counts(solver)):
         solver.set_tuning(0, grid)
         solver.set_tuning(1, xcd)
         solver.set_tuning(2, curve)

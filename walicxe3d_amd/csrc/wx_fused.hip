@@ -449,12 +449,12 @@ int fused_time_stages(FusedState &f, const DevCfg &c, hipStream_t st, int reps) 
 // kind 1: XCD-aware block order (1) or one range for all XCDs (0)
 // kind 2: block order along the Morton (0) or the Hilbert (1) curve
 // kind 3: FP32 MHD fluxes in delta form (0) or plain FP32 (1)
-// kind 4: z slabs per block (1, 2, 4, 8), one workgroup each, in the
-//         delta-form MHD kernels (by mesh size until set; no effect elsewhere)
+// kind 4: z slabs per block (1, 2, 4, 8, 16), one workgroup each, in the
+//         delta-form MHD kernels; 0, the default, by mesh size (no effect elsewhere)
 int fused_set_tuning(FusedState &f, int kind, int value) {
   if (kind < 0 || kind > 4) return 1;
   if ((kind == 2 || kind == 3) && (value < 0 || value > 1)) return 1;
-  if (kind == 4 && value != 1 && value != 2 && value != 4 && value != 8) return 1;
+  if (kind == 4 && (value < 0 || value > NC || (value & (value - 1)))) return 1;
   drop_graphs(f);
   if (kind == 3) {
     f.mhd_plain32 = value;
