@@ -6,13 +6,25 @@
 // <input>.blocks).  With EMU_VTK_DIR set, writeOutput's VTK files of the
 // initial and the final state (output numbers 0 and nsteps, one passive
 // column, units_type EMU_VTK_UNITS, default CODE_UNITS) go to that folder.
+// With EMU_COUNTS set, single calls on the final state are made as well, and
+// what each asked the runtime for is printed (device allocations, copies,
+// most device bytes alive).
 #include <cstdio>
 #include <cstdlib>
 #include <vector>
 #include <cstring>
 #include <string>
 #include "walicxe_hip.h"
+#include "hip/hip_runtime.h"
 static int run_case(const char *path, int nsteps);
+template <typename F> static int counted(const char *name, F call) {
+  const size_t m = emu_counts.mallocs, n = emu_counts.copies;
+  emu_counts.peak = emu_counts.live.load();
+  const int rc = call();
+  printf("count %s mallocs %zu copies %zu peak %zu\n", name, emu_counts.mallocs - m, emu_counts.copies - n, emu_counts.peak.load());
+  if (rc < 0) printf("%s %d %s\n", name, rc, wx_last_error());
+  return rc;
+}
 int main(int argc, char **argv) {
   for (int a = 1; a + 1 < argc; a += 2) {
     printf("case %s steps %s\n", argv[a], argv[a + 1]); fflush(stdout);
@@ -109,6 +121,11 @@ static int run_case(const char *path, int nsteps) {
   // (hydro with passives: the file's passive columns hold the carried ones)
   { const int np = (cfg.nv == 6 || cfg.nv == 7) ? cfg.nv - 5 : 1;
     std::string fn = std::string(path) + ".wxbin"; if (wx_write_bin(ctx, fn.c_str(), np) < 0) { printf("write_bin %s\n", wx_last_error()); return 1; } }
+  if (getenv("EMU_COUNTS")) {
+    double raw;
+    std::vector<double> P(U.size());
+    if (counted("get_timestep", [&] { return wx_get_timestep(ctx, &raw); }) < 0) return 1;
+  }
   double s = 0; for (double x : Uo) s += x;
   printf("it %d dt %.17g time %.17g sum %.17g\n", it, dt, time, s);
   wx_finalize(ctx);

@@ -6,6 +6,8 @@
 // reported with its source line.  Kernels run one workgroup at a time, each
 // lane a fiber (tests/emu/emu_rt.cpp); graphs are recorded and replayed.
 #pragma once
+#include <malloc.h>
+
 #include <atomic>
 #include <barrier>
 #include <cmath>
@@ -61,8 +63,23 @@ inline hipError_t hipGetDeviceCount(int *n) { *n = 1; return hipSuccess; }
 inline hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
 inline hipError_t hipSetDevice(int) { return hipSuccess; }
 inline hipError_t hipDeviceSynchronize() { return hipSuccess; }
-template <typename T> inline hipError_t hipMalloc(T **p, size_t n) { *p = (T *)malloc(n ? n : 1); return *p ? hipSuccess : 2; }
-inline hipError_t hipFree(void *p) { free(p); return hipSuccess; }
+// what the library asked the runtime for (device bytes alive and at most, calls)
+struct EmuCounts { std::atomic<size_t> live{0}, peak{0}, mallocs{0}, copies{0}; };
+inline EmuCounts emu_counts;
+template <typename T> inline hipError_t hipMalloc(T **p, size_t n) {
+  *p = (T *)malloc(n ? n : 1);
+  if (!*p) return 2;
+  emu_counts.mallocs++;
+  const size_t l = emu_counts.live += malloc_usable_size(*p);
+  size_t top = emu_counts.peak;
+  while (l > top && !emu_counts.peak.compare_exchange_weak(top, l)) {}
+  return hipSuccess;
+}
+inline hipError_t hipFree(void *p) {
+  if (p) emu_counts.live -= malloc_usable_size(p);
+  free(p);
+  return hipSuccess;
+}
 enum { hipHostMallocDefault = 0 };
 template <typename T> inline hipError_t hipHostMalloc(T **p, size_t n, unsigned) {
   *p = (T *)malloc(n ? n : 1);
@@ -73,6 +90,7 @@ inline hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { m
 
 void emu_record_or_run(hipStream_t st, std::function<void()> f);
 inline hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind, hipStream_t st = nullptr) {
+  emu_counts.copies++;
   emu_record_or_run(st, [=] { memcpy(d, s, n); });
   return hipSuccess;
 }

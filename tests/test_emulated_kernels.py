@@ -175,6 +175,26 @@ def test_z_slabs_leave_the_state_unchanged(emu, tmp_path):
             assert np.array_equal(o, outs[0]), w.name
 
 
+def _counts(emu, tmp, name, w, form, **env):
+    """Case `name` with EMU_COUNTS: {call: {mallocs, copies, peak}}."""
+    p = os.path.join(str(tmp), name + ".bin")
+    blocks, U0 = _write_input(p, w, form)
+    out = {}
+    for line in _run(emu, [p, "1"], str(tmp), EMU_COUNTS="1", **env).splitlines():
+        t = line.split()
+        if t and t[0] == "count":
+            out[t[1]] = {t[i]: int(t[i + 1]) for i in range(2, len(t), 2)}
+    return out, U0
+
+
+def test_fused_timestep_takes_one_transfer(emu, tmp_path):
+    """wx_get_timestep reads the step's scalars and the partial minima of dt
+    in one copy (a copy costs 12 us whatever its size)."""
+    for form in (hip.FUSED_FP32, hip.FUSED_FP64):
+        c, _ = _counts(emu, tmp_path, "dt%d" % form, W.get("blast_reflect"), form)
+        assert c["get_timestep"]["copies"] == 1 and c["get_timestep"]["mallocs"] == 0
+
+
 def test_slab_count_of_the_rule_can_be_set_and_given_back(emu, tmp_path):
     """Kind 4 takes every count the rule by mesh size can choose (16 on these
     8 blocks, viscous and inviscid) and 0 for the rule itself: the same state

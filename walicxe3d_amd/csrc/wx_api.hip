@@ -106,9 +106,10 @@ struct Ctx {
   double *d_tabT = nullptr, *d_tabC = nullptr;
   // plain form; dP and dP2 swap when a second stage's primitives replace the first's
   double *dU = nullptr, *dUP = nullptr, *dP = nullptr, *dP2 = nullptr;
+  // plain form: the step's scalars with the partial minima of dt, and behind
+  // them, in the same allocation, two words of single routines
+  StepRecord *d_rec = nullptr;
   unsigned long long *d_scal = nullptr;  // [0] dt bits, [1] floor count
-  unsigned long long *d_slots = nullptr; // plain form: partial minima of dt (DT_SLOTS)
-  StepState *d_ss = nullptr;             // plain form: the step's scalars
   bool have_state = false;
   bool ghosts_recorded = false;      // fused form: ghost layer of wx_record_ghosts in d_ghosts
   double *d_ghosts = nullptr;        // [blk][rho, p][6][256]
@@ -601,7 +602,7 @@ int to_host(Ctx *c, double *dst, const double *src, size_t n) {
 
 // ------------------------- plain-form sequences ----------------------------
 int plain_timestep_raw(Ctx *c, double *dt) {
-  plain_timestep(c->dc, c->dP, c->d_slots, c->d_scal, c->st);
+  plain_timestep(c->dc, c->dP, c->d_rec->slots, c->d_scal, c->st);
   unsigned long long bits = 0;
   HIPCHK(hipMemcpyAsync(&bits, c->d_scal, sizeof(bits), hipMemcpyDeviceToHost, c->st));
   HIPCHK(hipStreamSynchronize(c->st));
@@ -645,15 +646,15 @@ int plain_steps(Ctx *c, int nsteps, int *it, double *dt, double *time, int *next
   s.nextout = *nextout;
   s.dtout = dtout;
   s.t_sc = t_sc;
-  HIPCHK(hipMemcpyAsync(c->d_ss, &s, sizeof(s), hipMemcpyHostToDevice, c->st));
+  HIPCHK(hipMemcpyAsync(&c->d_rec->s, &s, sizeof(s), hipMemcpyHostToDevice, c->st));
   for (int n = 0; n < nsteps; n++) {
-    plain_step_begin(c->dc, n == 0 ? c->dP : nullptr, c->d_ss, c->d_slots, c->st);
-    plain_stages(c, c->cfg.solver == SOLVER_HLL1 ? 1 : 2, c->d_ss, 0.0);
-    plain_finish(c->dc, c->dUP, c->dU, c->dP, c->d_ss, c->cfg.mu0, n + 1 < nsteps ? c->d_slots : nullptr, c->st);
+    plain_step_begin(c->dc, n == 0 ? c->dP : nullptr, &c->d_rec->s, c->d_rec->slots, c->st);
+    plain_stages(c, c->cfg.solver == SOLVER_HLL1 ? 1 : 2, &c->d_rec->s, 0.0);
+    plain_finish(c->dc, c->dUP, c->dU, c->dP, &c->d_rec->s, c->cfg.mu0, n + 1 < nsteps ? c->d_rec->slots : nullptr, c->st);
   }
   int rc = launch_check("step");
   if (rc != WX_OK) return rc;
-  HIPCHK(hipMemcpyAsync(&s, c->d_ss, sizeof(s), hipMemcpyDeviceToHost, c->st));
+  HIPCHK(hipMemcpyAsync(&s, &c->d_rec->s, sizeof(s), hipMemcpyDeviceToHost, c->st));
   HIPCHK(hipStreamSynchronize(c->st));
   step_close(&s);
   *it = s.it;
@@ -1040,16 +1041,15 @@ int wx_init(const wx_config *cfg, void **out) {
     delete c;
     return fail(WX_EHIP, "stream creation failed");
   }
-  const size_t slot_bytes = DT_SLOTS * DT_STRIDE * sizeof(unsigned long long);
-  if (hipMalloc(&c->d_scal, 4 * sizeof(unsigned long long)) != hipSuccess ||
-      hipMalloc(&c->d_slots, slot_bytes) != hipSuccess || hipMalloc(&c->d_ss, sizeof(StepState)) != hipSuccess ||
-      hipMemsetAsync(c->d_slots, 0xFF, slot_bytes, c->st) != hipSuccess) {
-    hipFree(c->d_scal);
-    hipFree(c->d_slots);
-    hipFree(c->d_ss);
-    hipStreamDestroy(c->st);
-    delete c;
-    return fail(WX_ENOMEM, "device allocation failed");
+  if (!is_fused(c)) {
+    if (hipMalloc(&c->d_rec, sizeof(StepRecord) + 2 * sizeof(unsigned long long)) != hipSuccess ||
+        hipMemsetAsync(c->d_rec->slots, 0xFF, sizeof(c->d_rec->slots), c->st) != hipSuccess) {
+      hipFree(c->d_rec);
+      hipStreamDestroy(c->st);
+      delete c;
+      return fail(WX_ENOMEM, "device allocation failed");
+    }
+    c->d_scal = reinterpret_cast<unsigned long long *>(c->d_rec + 1);
   }
   if (cfg->cooling) {
     hipMalloc(&c->d_tabT, sizeof(double) * cfg->ntab);
@@ -1068,9 +1068,7 @@ int wx_finalize(void *ctx) {
   if (!c) return WX_OK;
   hipStreamSynchronize(c->st);
   free_mesh(c);
-  hipFree(c->d_scal);
-  hipFree(c->d_slots);
-  hipFree(c->d_ss);
+  hipFree(c->d_rec);
   hipFree(c->d_tabT);
   hipFree(c->d_tabC);
   hipFree(c->d_stage);

@@ -50,6 +50,13 @@ struct StepState {
 // words over which workgroups spread the smallest dt (one per 64-byte line)
 constexpr int DT_SLOTS = 64, DT_STRIDE = 8;
 
+// Both in one allocation, so that one transfer moves them; the slots start on
+// a line of their own (every workgroup reads dt while others update a slot).
+struct StepRecord {
+  StepState s;
+  alignas(256) unsigned long long slots[DT_SLOTS * DT_STRIDE];
+};
+
 // dt of a step from the smallest dx/(|v|+c): CFL, start-up ramp, output
 // clamp (source/hydro_solver.f90:183-207)
 __device__ inline void step_open(StepState *s, double m, double cfl, int cooling) {

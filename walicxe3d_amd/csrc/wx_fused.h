@@ -21,11 +21,10 @@ struct FusedState {
   // the state between the second stage and the end of the step, where that is
   // a kernel of its own (hydro, FP64, viscous FP32 MHD)
   double *X = nullptr;
-  unsigned long long *slots = nullptr;   // partial minima of dt, next to step's dtmin_bits
   void *UP = nullptr;        // [blk][nv][4096] half-step state (FP32, or FP64 in the fp64 variant)
   int fp64 = 0;              // flux arithmetic and UP storage in FP64
   int *order = nullptr;      // block processing order (device)
-  StepState *step = nullptr; // device
+  StepRecord *rec = nullptr; // device: the step's scalars and the partial minima of dt
   int nblk = 0, nv = 0;
   int grid = 0;              // stage-kernel grid size (0 = one workgroup per block)
   int xcd_map = 1;           // XCD-aware block order

@@ -160,9 +160,8 @@ int fused_alloc(FusedState &f, const DevCfg &c, const std::vector<BlockInfo> &in
   if (f.two_u) FCHK(hipMalloc(&f.U2, n * sizeof(double)));
   FCHK(hipMalloc(&f.UP, n * (f.fp64 ? sizeof(double) : sizeof(float))));
   FCHK(hipMalloc(&f.order, c.nblk * sizeof(int)));
-  FCHK(hipMalloc(&f.step, sizeof(StepState)));
+  FCHK(hipMalloc(&f.rec, sizeof(StepRecord)));
   if (!f.two_u || ends_apart(c)) FCHK(hipMalloc(&f.X, n * sizeof(double)));
-  FCHK(hipMalloc(&f.slots, DT_SLOTS * DT_STRIDE * sizeof(unsigned long long)));
   f.host_info = info;
   f.maxlev = c.maxlev;
   if (build_order(f)) return 1;
@@ -187,9 +186,8 @@ void fused_free(FusedState &f) {
   hipFree(f.U2);
   hipFree(f.UP);
   hipFree(f.order);
-  hipFree(f.step);
+  hipFree(f.rec);
   hipFree(f.X);
-  hipFree(f.slots);
   for (int e = 0; e < 4; e++)
     if (f.ev[e]) hipEventDestroy(f.ev[e]);
   for (int e = 0; e < 4; e++) f.ev[e] = nullptr;
@@ -197,9 +195,8 @@ void fused_free(FusedState &f) {
   f.U2 = nullptr;
   f.UP = nullptr;
   f.order = nullptr;
-  f.step = nullptr;
+  f.rec = nullptr;
   f.X = nullptr;
-  f.slots = nullptr;
 }
 
 static FusedArgs make_args(FusedState &f, const DevCfg &c) {
@@ -210,9 +207,9 @@ static FusedArgs make_args(FusedState &f, const DevCfg &c) {
   a.UPin = f.UP;
   a.UPout = f.UP;
   a.X = f.X;
-  a.slots = f.slots;
+  a.slots = f.rec->slots;
   a.order = f.order;
-  a.step = f.step;
+  a.step = &f.rec->s;
   a.nblk = f.nblk;
   a.nslab = 1;
   return a;
@@ -231,10 +228,10 @@ int fused_upload(FusedState &f, const DevCfg &c, double *U, bool adopt, hipStrea
   } else {
     FCHK(hipMemcpyAsync(f.U, U, (size_t)f.nblk * f.nv * NINT * sizeof(double), hipMemcpyDeviceToDevice, st));
   }
-  StepState s{};
-  s.dtmin_bits = ~0ull;
-  FCHK(hipMemcpyAsync(f.step, &s, sizeof(s), hipMemcpyHostToDevice, st));
-  FCHK(hipMemsetAsync(f.slots, 0xFF, DT_SLOTS * DT_STRIDE * sizeof(unsigned long long), st));
+  StepRecord r{};
+  r.s.dtmin_bits = ~0ull;
+  std::memset(r.slots, 0xFF, sizeof(r.slots));
+  FCHK(hipMemcpyAsync(f.rec, &r, sizeof(r), hipMemcpyHostToDevice, st));
   launch_dt_init(f, c, st);
   FCHK(hipGetLastError());
   FCHK(hipStreamSynchronize(st));
@@ -253,16 +250,15 @@ int fused_prims(FusedState &f, const DevCfg &c, double *P, hipStream_t st) {
 }
 
 int fused_timestep(FusedState &f, const DevCfg &c, hipStream_t st, double *dt_raw) {
-  StepState s;
-  unsigned long long slots[DT_SLOTS * DT_STRIDE];
-  FCHK(hipMemcpyAsync(&s, f.step, sizeof(s), hipMemcpyDeviceToHost, st));
-  FCHK(hipMemcpyAsync(slots, f.slots, sizeof(slots), hipMemcpyDeviceToHost, st));
+  // one transfer: two took 37 us, one 25
+  StepRecord r;
+  FCHK(hipMemcpyAsync(&r, f.rec, sizeof(r), hipMemcpyDeviceToHost, st));
   FCHK(hipStreamSynchronize(st));
   // an untouched word reads as a NaN, which fmin drops
   double m, q;
-  std::memcpy(&m, &s.dtmin_bits, sizeof(m));
+  std::memcpy(&m, &r.s.dtmin_bits, sizeof(m));
   for (int n = 0; n < DT_SLOTS; n++) {
-    std::memcpy(&q, &slots[n * DT_STRIDE], sizeof(q));
+    std::memcpy(&q, &r.slots[n * DT_STRIDE], sizeof(q));
     m = std::fmin(m, q);
   }
   *dt_raw = c.cooling ? std::fmin(m, 1.0e30) * c.cfl : m * c.cfl;
@@ -341,7 +337,7 @@ static void launch_rest(FusedState &f, const DevCfg &c, hipStream_t st) {
 }
 
 static void enqueue_step(FusedState &f, const DevCfg &c, hipStream_t st) {
-  hipLaunchKernelGGL(k_begin, dim3(1), dim3(64), 0, st, f.step, f.slots, c.cfl, c.cooling);
+  hipLaunchKernelGGL(k_begin, dim3(1), dim3(64), 0, st, &f.rec->s, f.rec->slots, c.cfl, c.cooling);
   launch_stage(f, c, st, 1);
   launch_stage(f, c, st, 2);
   launch_rest(f, c, st);
@@ -388,7 +384,7 @@ int fused_run(FusedState &f, const DevCfg &c, hipStream_t st, int nsteps, int *i
   if (nsteps == 0) return 0;
   // host scalars -> device (keeps the running dt minimum)
   StepState s;
-  FCHK(hipMemcpyAsync(&s, f.step, sizeof(s), hipMemcpyDeviceToHost, st));
+  FCHK(hipMemcpyAsync(&s, &f.rec->s, sizeof(s), hipMemcpyDeviceToHost, st));
   FCHK(hipStreamSynchronize(st));
   s.it = *it;
   s.time = *time;
@@ -396,7 +392,7 @@ int fused_run(FusedState &f, const DevCfg &c, hipStream_t st, int nsteps, int *i
   s.dtout = dtout;
   s.t_sc = t_sc;
   s.open = 0;
-  FCHK(hipMemcpyAsync(f.step, &s, sizeof(s), hipMemcpyHostToDevice, st));
+  FCHK(hipMemcpyAsync(&f.rec->s, &s, sizeof(s), hipMemcpyHostToDevice, st));
   hipGraphExec_t ex[2];
   if (step_graphs(f, c, st, ex)) return 1;
   FCHK(hipEventRecord(f.ev[0], st));
@@ -405,7 +401,7 @@ int fused_run(FusedState &f, const DevCfg &c, hipStream_t st, int nsteps, int *i
     swap_u(f);
   }
   FCHK(hipEventRecord(f.ev[1], st));
-  FCHK(hipMemcpyAsync(&s, f.step, sizeof(s), hipMemcpyDeviceToHost, st));
+  FCHK(hipMemcpyAsync(&s, &f.rec->s, sizeof(s), hipMemcpyDeviceToHost, st));
   FCHK(hipStreamSynchronize(st));
   float ms = 0;
   hipEventElapsedTime(&ms, f.ev[0], f.ev[1]);
@@ -423,7 +419,7 @@ int fused_run(FusedState &f, const DevCfg &c, hipStream_t st, int nsteps, int *i
 int fused_time_stages(FusedState &f, const DevCfg &c, hipStream_t st, int reps) {
   float a1 = 0, a2 = 0;
   for (int r = 0; r < reps; r++) {
-    hipLaunchKernelGGL(k_begin, dim3(1), dim3(64), 0, st, f.step, f.slots, c.cfl, c.cooling);
+    hipLaunchKernelGGL(k_begin, dim3(1), dim3(64), 0, st, &f.rec->s, f.rec->slots, c.cfl, c.cooling);
     FCHK(hipEventRecord(f.ev[0], st));
     launch_stage(f, c, st, 1);
     FCHK(hipEventRecord(f.ev[1], st));
