@@ -125,6 +125,10 @@ static int run_case(const char *path, int nsteps) {
     double raw;
     std::vector<double> P(U.size());
     if (counted("get_timestep", [&] { return wx_get_timestep(ctx, &raw); }) < 0) return 1;
+    if (counted("download", [&] { return wx_download_state(ctx, U.data(), P.data(), WX_LAYOUT_BLOCKS, 0, nullptr); }) < 0) return 1;
+    if (counted("upload", [&] { return wx_upload_state(ctx, Uo.data(), WX_LAYOUT_BLOCKS, 0, nullptr); }) < 0) return 1;
+    if (counted("remesh", [&] { return wx_remesh(ctx, nblk, bids.data()); }) < 0) return 1;
+    if (cfg.form != WX_FORM_PLAIN_FP64 && counted("run", [&] { return wx_run(ctx, 1, &it, &dt, &time, &nextout, dtout_tsc[0], dtout_tsc[1]); }) < 0) return 1;
   }
   double s = 0; for (double x : Uo) s += x;
   printf("it %d dt %.17g time %.17g sum %.17g\n", it, dt, time, s);

@@ -195,6 +195,25 @@ def test_fused_timestep_takes_one_transfer(emu, tmp_path):
         assert c["get_timestep"]["copies"] == 1 and c["get_timestep"]["mallocs"] == 0
 
 
+# bytes per variable and zone that a form holds with U, UP (and U2) and an
+# upload's or a mesh change's buffer
+@pytest.mark.parametrize("name,form,held", [
+    ("blast_reflect", hip.FUSED_FP32, 20), ("blast_reflect", hip.FUSED_FP64, 24), ("mhd_hlle", hip.FUSED_FP32, 28),
+    ("mhd_hlle", hip.FUSED_FP64, 24)])
+def test_no_call_holds_a_state_more_than_an_upload(emu, tmp_path, name, form, held):
+    """The state between the second stage and the end of the step takes no
+    room beside an upload's staging buffer, the primitives of a download or
+    the two states of a mesh change: the largest mesh that a run takes is the
+    largest that an upload takes.  4 kB a block stand for its tables, 64 kB
+    for what does not grow with the mesh (a state is 0.8 MB or more here)."""
+    w = W.get(name)
+    c, U0 = _counts(emu, tmp_path, "mem%s%d" % (name, form), w, form)
+    one = U0.size
+    lim = held * one + 4096 * len(U0) + 65536
+    for call in ("download", "upload", "remesh", "run"):
+        assert c[call]["peak"] <= lim, (call, c[call]["peak"] / one)
+
+
 def test_slab_count_of_the_rule_can_be_set_and_given_back(emu, tmp_path):
     """Kind 4 takes every count the rule by mesh size can choose (16 on these
     8 blocks, viscous and inviscid) and 0 for the rule itself: the same state

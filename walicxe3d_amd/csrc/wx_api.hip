@@ -1082,9 +1082,10 @@ int wx_finalize(void *ctx) {
 
 // wx_set_mesh; `pre`, when given, holds the face table of this block list
 // already built (check_mesh with the context's nroot, maxlev and boundaries),
-// which is taken over instead of built again
+// which is taken over instead of built again; adopt: an upload_device that
+// adopts its buffer follows
 static int set_mesh_impl(Ctx *c, const int nroot[3], int maxlev, const double *dxyz, int nblk, const int *bids,
-                         Ctx *pre) {
+                         Ctx *pre, bool adopt = false) {
   HIPCHK(hipStreamSynchronize(c->st));
   free_mesh(c);
   c->nblk = nblk;
@@ -1118,7 +1119,7 @@ static int set_mesh_impl(Ctx *c, const int nroot[3], int maxlev, const double *d
   if (is_fused(c)) {
     c->fused.fp64 = c->cfg.form == WX_FORM_FUSED_FP64;
     for (int d = 0; d < 3; d++) c->fused.nroot[d] = c->nroot[d];
-    int frc = fused_alloc(c->fused, c->dc, c->info, c->st);
+    int frc = fused_alloc(c->fused, c->dc, c->info, adopt, c->st);
     if (frc != 0) return fail(WX_ENOMEM, "fused-form allocation failed");
   }
   return WX_OK;
@@ -1168,14 +1169,18 @@ int wx_upload_state(void *ctx, const double *u, int layout, int nbmax, const int
     return fail(WX_EINVAL, "unknown layout");
   }
   DevBuf<double> d_in;
-  HIPCHK(d_in.alloc(ni));
+  double *in = is_fused(c) ? c->fused.X : nullptr;   // nothing in it between runs
+  if (!in) {
+    HIPCHK(d_in.alloc(ni));
+    in = d_in.p;
+  }
   if (layout == WX_LAYOUT_FORTRAN) {
-    int rc = fortran_stage_in(c, u, d_in.p, nbmax, lb);
+    int rc = fortran_stage_in(c, u, in, nbmax, lb);
     if (rc != WX_OK) return rc;
   } else {
-    HIPCHK(hipMemcpyAsync(d_in.p, u, ni * sizeof(double), hipMemcpyHostToDevice, c->st));
+    HIPCHK(hipMemcpyAsync(in, u, ni * sizeof(double), hipMemcpyHostToDevice, c->st));
   }
-  return upload_device(c, d_in.p);
+  return upload_device(c, in);
 }
 
 int wx_upload_prims(void *ctx, const double *p, int layout, int nbmax, const int *lb) {
@@ -1227,8 +1232,11 @@ int wx_download_state(void *ctx, double *u, double *prim, int layout, int nbmax,
       // the fused state is already in the block layout of the interface
       from = c->fused.U;
     } else {
-      if (!d_out.p) HIPCHK(d_out.alloc(ni));
-      double *out = d_out.p;
+      double *out = is_fused(c) ? c->fused.X : nullptr;   // nothing in it between runs
+      if (!out) {
+        if (!d_out.p) HIPCHK(d_out.alloc(ni));
+        out = d_out.p;
+      }
       if (is_fused(c)) {
         if (fused_prims(c->fused, c->dc, out, c->st)) return fail(WX_EHIP, fused_error());
       } else {
@@ -1405,6 +1413,7 @@ static int remesh_impl(Ctx *c, int nblk, const int *bids, Ctx *pre) {
     // state is remapped straight from it and becomes the new fused state
     DevBuf<double> d_new;
     DevBuf<RemapSrc> d_map;
+    fused_drop_x(c->fused);
     HIPCHK(d_new.alloc(nnew));
     HIPCHK(d_map.alloc(table.size()));
     HIPCHK(hipMemcpyAsync(d_map.p, table.data(), table.size() * sizeof(RemapSrc), hipMemcpyHostToDevice, c->st));
@@ -1416,7 +1425,7 @@ static int remesh_impl(Ctx *c, int nblk, const int *bids, Ctx *pre) {
     if (rc == WX_OK) {
       const std::vector<double> dxyz = c->dxyz;
       int nroot[3] = {c->nroot[0], c->nroot[1], c->nroot[2]};
-      rc = set_mesh_impl(c, nroot, c->maxlev, dxyz.data(), nblk, bids, pre);
+      rc = set_mesh_impl(c, nroot, c->maxlev, dxyz.data(), nblk, bids, pre, true);
     }
     if (rc != WX_OK) return rc;
     return upload_device(c, d_new.release(), true);   // the fused state owns it now

@@ -19,7 +19,8 @@ struct FusedState {
   double *U2 = nullptr;
   int two_u = 0;
   // the state between the second stage and the end of the step, where that is
-  // a kernel of its own (hydro, FP64, viscous FP32 MHD)
+  // a kernel of its own (hydro, FP64, viscous or cooling FP32 MHD).  It is
+  // there from the first run on; between runs a transfer may use it.
   double *X = nullptr;
   void *UP = nullptr;        // [blk][nv][4096] half-step state (FP32, or FP64 in the fp64 variant)
   int fp64 = 0;              // flux arithmetic and UP storage in FP64
@@ -45,8 +46,11 @@ struct FusedState {
   int maxlev = 0;
 };
 
-int fused_alloc(FusedState &f, const DevCfg &c, const std::vector<BlockInfo> &info, hipStream_t st);
+// Arrays for a mesh; adopt: without the state, which fused_upload will adopt.
+int fused_alloc(FusedState &f, const DevCfg &c, const std::vector<BlockInfo> &info, bool adopt, hipStream_t st);
 void fused_free(FusedState &f);
+// X given back (allocated again by the next run)
+void fused_drop_x(FusedState &f);
 // State in from U ([blk][nv][16^3] FP64, device): copied, or with adopt the
 // buffer itself becomes the state (the library frees it); dt re-initialised.
 int fused_upload(FusedState &f, const DevCfg &c, double *U, bool adopt, hipStream_t st);

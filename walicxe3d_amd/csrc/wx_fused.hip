@@ -150,18 +150,17 @@ static int build_order(FusedState &f) {
   return 0;
 }
 
-int fused_alloc(FusedState &f, const DevCfg &c, const std::vector<BlockInfo> &info, hipStream_t st) {
+int fused_alloc(FusedState &f, const DevCfg &c, const std::vector<BlockInfo> &info, bool adopt, hipStream_t st) {
   fused_free(f);
   f.nblk = c.nblk;
   f.nv = c.nv;
   f.two_u = !f.fp64 && c.nv == 8;
   size_t n = (size_t)c.nblk * c.nv * NINT;
-  FCHK(hipMalloc(&f.U, n * sizeof(double)));
+  if (!adopt) FCHK(hipMalloc(&f.U, n * sizeof(double)));
   if (f.two_u) FCHK(hipMalloc(&f.U2, n * sizeof(double)));
   FCHK(hipMalloc(&f.UP, n * (f.fp64 ? sizeof(double) : sizeof(float))));
   FCHK(hipMalloc(&f.order, c.nblk * sizeof(int)));
   FCHK(hipMalloc(&f.rec, sizeof(StepRecord)));
-  if (!f.two_u || ends_apart(c)) FCHK(hipMalloc(&f.X, n * sizeof(double)));
   f.host_info = info;
   f.maxlev = c.maxlev;
   if (build_order(f)) return 1;
@@ -178,6 +177,23 @@ static void drop_graphs(FusedState &f) {
   f.exec = f.exec2 = nullptr;
   f.graph = f.graph2 = nullptr;
   f.graph_u = f.graph2_u = nullptr;
+}
+
+void fused_drop_x(FusedState &f) {
+  if (!f.X) return;
+  drop_graphs(f);
+  hipFree(f.X);
+  f.X = nullptr;
+}
+
+// X comes with the first run: an upload's staging buffer and the two states of
+// a mesh change, each as large, are gone by then, so the largest mesh that
+// fits is the one that it was without X (hydro FP32: 20 bytes a variable and
+// zone at most, in an upload, a mesh change and a run alike).
+static int need_x(FusedState &f, const DevCfg &c) {
+  if (f.X || (f.two_u && !ends_apart(c))) return 0;
+  FCHK(hipMalloc(&f.X, (size_t)f.nblk * f.nv * NINT * sizeof(double)));
+  return 0;
 }
 
 void fused_free(FusedState &f) {
@@ -226,7 +242,9 @@ int fused_upload(FusedState &f, const DevCfg &c, double *U, bool adopt, hipStrea
     hipFree(f.U);
     f.U = U;
   } else {
-    FCHK(hipMemcpyAsync(f.U, U, (size_t)f.nblk * f.nv * NINT * sizeof(double), hipMemcpyDeviceToDevice, st));
+    const size_t bytes = (size_t)f.nblk * f.nv * NINT * sizeof(double);
+    if (!f.U) FCHK(hipMalloc(&f.U, bytes));   // an adoption that failed
+    FCHK(hipMemcpyAsync(f.U, U, bytes, hipMemcpyDeviceToDevice, st));
   }
   StepRecord r{};
   r.s.dtmin_bits = ~0ull;
@@ -382,6 +400,7 @@ static int step_graphs(FusedState &f, const DevCfg &c, hipStream_t st, hipGraphE
 int fused_run(FusedState &f, const DevCfg &c, hipStream_t st, int nsteps, int *it, double *dt, double *time,
               int *nextout, double dtout, double t_sc) {
   if (nsteps == 0) return 0;
+  if (need_x(f, c)) return 1;
   // host scalars -> device (keeps the running dt minimum)
   StepState s;
   FCHK(hipMemcpyAsync(&s, &f.rec->s, sizeof(s), hipMemcpyDeviceToHost, st));
@@ -418,6 +437,7 @@ int fused_run(FusedState &f, const DevCfg &c, hipStream_t st, int nsteps, int *i
 // by replaying one step outside the graph; used by the benchmark.
 int fused_time_stages(FusedState &f, const DevCfg &c, hipStream_t st, int reps) {
   float a1 = 0, a2 = 0;
+  if (need_x(f, c)) return 1;
   for (int r = 0; r < reps; r++) {
     hipLaunchKernelGGL(k_begin, dim3(1), dim3(64), 0, st, &f.rec->s, f.rec->slots, c.cfl, c.cooling);
     FCHK(hipEventRecord(f.ev[0], st));
