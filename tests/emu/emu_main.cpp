@@ -126,6 +126,12 @@ static int run_case(const char *path, int nsteps) {
     std::vector<double> P(U.size());
     if (counted("get_timestep", [&] { return wx_get_timestep(ctx, &raw); }) < 0) return 1;
     if (counted("download", [&] { return wx_download_state(ctx, U.data(), P.data(), WX_LAYOUT_BLOCKS, 0, nullptr); }) < 0) return 1;
+    if (counted("plain_host", [&] { return wx_download_state(ctx, U.data(), nullptr, WX_LAYOUT_BLOCKS, 0, nullptr); }) < 0) return 1;
+    emu_pinned = P.data();
+    emu_pinned_bytes = 8 * P.size();
+    if (counted("pinned_host", [&] { return wx_download_state(ctx, P.data(), nullptr, WX_LAYOUT_BLOCKS, 0, nullptr); }) < 0) return 1;
+    emu_pinned = nullptr;
+    printf("pinned and plain %s\n", P == U ? "agree" : "differ");
     if (counted("upload", [&] { return wx_upload_state(ctx, Uo.data(), WX_LAYOUT_BLOCKS, 0, nullptr); }) < 0) return 1;
     if (counted("remesh", [&] { return wx_remesh(ctx, nblk, bids.data()); }) < 0) return 1;
     if (cfg.form != WX_FORM_PLAIN_FP64 && counted("run", [&] { return wx_run(ctx, 1, &it, &dt, &time, &nextout, dtout_tsc[0], dtout_tsc[1]); }) < 0) return 1;

@@ -81,11 +81,21 @@ inline hipError_t hipFree(void *p) {
   return hipSuccess;
 }
 enum { hipHostMallocDefault = 0 };
+// one range that hipPointerGetAttributes knows as pinned
+inline void *emu_pinned;
+inline size_t emu_pinned_bytes;
 template <typename T> inline hipError_t hipHostMalloc(T **p, size_t n, unsigned) {
   *p = (T *)malloc(n ? n : 1);
   return *p ? hipSuccess : 2;
 }
 inline hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
+enum { hipMemoryTypeUnregistered = 0, hipMemoryTypeHost = 1 };
+struct hipPointerAttribute_t { int type; };
+inline hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p) {
+  const char *q = (const char *)p, *b = (const char *)emu_pinned;
+  a->type = b && q >= b && q < b + emu_pinned_bytes ? hipMemoryTypeHost : hipMemoryTypeUnregistered;
+  return hipSuccess;
+}
 inline hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind) { memcpy(d, s, n); return hipSuccess; }
 
 void emu_record_or_run(hipStream_t st, std::function<void()> f);

@@ -214,6 +214,16 @@ def test_no_call_holds_a_state_more_than_an_upload(emu, tmp_path, name, form, he
         assert c[call]["peak"] <= lim, (call, c[call]["peak"] / one)
 
 
+def test_pinned_destinations_are_copied_to_directly(emu, tmp_path):
+    """A download of 10 MB goes through the lanes' chunks to ordinary memory
+    and in one copy to memory that the caller pinned."""
+    w = W.get("sedov")
+    c, U0 = _counts(emu, tmp_path, "pinned", w, hip.FUSED_FP32)
+    assert U0.nbytes > (8 << 20)
+    assert c["plain_host"]["copies"] == -(-U0.nbytes // (1 << 20))
+    assert c["pinned_host"]["copies"] == 1
+
+
 def test_slab_count_of_the_rule_can_be_set_and_given_back(emu, tmp_path):
     """Kind 4 takes every count the rule by mesh size can choose (16 on these
     8 blocks, viscous and inviscid) and 0 for the rule itself: the same state

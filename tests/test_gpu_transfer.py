@@ -65,3 +65,19 @@ def test_two_threads_and_a_new_context():
     assert np.array_equal(s.download(prim=False), U)
     assert np.array_equal(s.raw(0)[:, :, 2:18, 2:18, 2:18], U)
     s.close()
+
+
+def test_download_into_pinned_memory():
+    """Memory that the caller pinned takes the state directly (no chunks), at a
+    size that ordinary memory takes in chunks; also from its middle on."""
+    import ctypes as C
+    import torch
+    w, U = _state((13, 7, 1), 6)
+    s = hip.Walicxe3D(w, form=hip.FUSED_FP32)
+    s.upload(U)
+    for off in (0, 3):
+        pin = torch.zeros(U.size + off, dtype=torch.float64, pin_memory=True)
+        at = C.cast(pin.data_ptr() + 8 * off, hip._dp)
+        assert hip.load().wx_download_state(s._h, at, None, hip.LAYOUT_BLOCKS, 0, None) == 0
+        assert np.array_equal(pin.numpy()[off:].reshape(U.shape), U) and not pin[:off].any()
+    s.close()

@@ -563,11 +563,24 @@ hipError_t lane_copy(Ctx *c, int lane, size_t chunk, char *dst, const char *src,
   return e;
 }
 
+// ordinary host memory, that the runtime would stage itself; what the caller
+// pinned, managed or device memory it copies to directly (pinned: 1.5 ms for
+// 84 MB, against 2.2 through the lanes), and the lanes' memcpy has no business
+// in the last
+bool pageable(const void *p) {
+  hipPointerAttribute_t a;
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {   // memory the runtime does not know
+    (void)hipGetLastError();
+    return true;
+  }
+  return a.type == hipMemoryTypeUnregistered;
+}
+
 // n doubles on the device, ready in stream order, to host memory
 int to_host(Ctx *c, double *dst, const double *src, size_t n) {
   const size_t bytes = n * sizeof(double);
   std::unique_lock<std::mutex> use(g_lanes.busy, std::defer_lock);
-  if (bytes >= HOST_MIN && use.try_lock()) {
+  if (bytes >= HOST_MIN && pageable(dst) && use.try_lock()) {
     const size_t chunk = host_chunk(bytes);
     if (g_lanes.grow(2 * HOST_LANES * chunk)) {
       hipError_t err[HOST_LANES];
