@@ -1121,12 +1121,13 @@ static int set_mesh_impl(Ctx *c, const int nroot[3], int maxlev, const double *d
     // the plain form's arrays with ghost layers; the fused form keeps its
     // state without ghosts (FusedState) and needs none of them
     HIPCHK(hipMalloc(&c->dU, n * sizeof(double)));
-    HIPCHK(hipMalloc(&c->dP, n * sizeof(double)));
+    // P and P2 have room for 20^3 cubes (wx_copy_raw)
+    const size_t cubes = (size_t)nblk * c->cfg.nv * NCELL;
+    HIPCHK(hipMalloc(&c->dP, cubes * sizeof(double)));
     HIPCHK(hipMemset(c->dP, 0, n * sizeof(double)));
     HIPCHK(hipMalloc(&c->dUP, n * sizeof(double)));
     HIPCHK(hipMemset(c->dUP, 0, n * sizeof(double)));
-    HIPCHK(hipMalloc(&c->dP2, n * sizeof(double)));
-    HIPCHK(hipMemsetAsync(c->dP2, 0, n * sizeof(double), c->st));
+    HIPCHK(hipMalloc(&c->dP2, cubes * sizeof(double)));   // each use writes all of it before it is read
   }
   fill_devcfg(c, dxyz);
   if (is_fused(c)) {
@@ -1376,9 +1377,7 @@ int wx_copy_raw(void *ctx, int which, double *out) {
   if (is_fused(c)) return fail(WX_EINVAL, "plain-form entry point");
   const double *src = which == 0 ? c->dU : which == 1 ? c->dUP : c->dP;
   const size_t cubes = (size_t)c->nblk * c->cfg.nv, n = cubes * NCELL;
-  DevBuf<double> d_out;
-  HIPCHK(d_out.alloc(n));
-  double *to = d_out.p;
+  double *to = c->dP2;   // nothing in it between calls
   hipLaunchKernelGGL(k_cubes, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->st, cubes, src, to);
   rc = to_host(c, out, to, n);
   return rc != WX_OK ? rc : launch_check("copy_raw");

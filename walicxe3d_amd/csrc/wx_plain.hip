@@ -13,6 +13,9 @@ namespace wx {
 // step: 1053, 1008, 963, 978 us for 512, 1024, 2048, 4096; 512 hydro blocks:
 // 610, 538, 533, 534 us; 64 hydro blocks: 85, 81, 82, 82 us.
 constexpr int WX_UPDATE_WANT = 2048;
+// The same for the timestep pass (one column of 16 planes per lane is a serial
+// chain on a mesh of few blocks).
+constexpr int WX_TIMESTEP_WANT = 512;
 
 // ---------------------------------------------------------------------------
 // The device physics routines applied to arrays of records (one thread per
@@ -529,22 +532,23 @@ __device__ __forceinline__ void dt_to_slot(double dt, int slot, unsigned long lo
 }
 
 template <int NV>
-__global__ void __launch_bounds__(256) k_timestep(DevCfg c, const double *P, unsigned long long *slots) {
-  const int b = blockIdx.x, l = c.info[b].level - 1;
+__global__ void __launch_bounds__(256) k_timestep(DevCfg c, const double *P, unsigned long long *slots, int L) {
+  const int ns = NC / L, b = blockIdx.x / ns, k0 = blockIdx.x % ns * L + 1;
+  const int l = c.info[b].level - 1;
   const int i = threadIdx.x % NC + 1, j = threadIdx.x / NC + 1;
   const double dx = c.dx[0][l], dy = c.dx[1][l], dz = c.dx[2][l];
   constexpr int NP = NV == 8 ? 8 : 5;   // passive scalars don't enter
   const double *Pb = P + (size_t)b * NV * NSTORE;
   double dt = 1.0e30;
 #pragma unroll 2
-  for (int k = 1; k <= NC; k++) {
+  for (int k = k0; k < k0 + L; k++) {
     const int q = cid(i, j, k);
     double p[MAXV];
 #pragma unroll
     for (int v = 0; v < NP; v++) p[v] = Pb[v * NSTORE + q];
     dt = fmin(dt, dt_of<NV>(c, p, dx, dy, dz));
   }
-  dt_to_slot(dt, b, slots);
+  dt_to_slot(dt, blockIdx.x, slots);
 }
 
 // ---------------------------------------------------------------------------
@@ -692,13 +696,22 @@ __global__ void __launch_bounds__(256) k_mark(DevCfg c, const double *P, double 
   double m = 0.0;
   for (int s = 0; s < 2; s++) {
     const double *A = P + ((size_t)b * c.nv + (s == 0 ? 4 : 0)) * NSTORE;
-    for (int k = 1; k <= NC; k++) {
-      const int q = cid(i, j, k);
-      const double a = A[q];
-      const double gx = fabs(A[cid(i + 1, j, k)] - A[cid(i - 1, j, k)]) / a / two_dx;
-      const double gy = fabs(A[cid(i, j + 1, k)] - A[cid(i, j - 1, k)]) / a / two_dx;
-      const double gz = fabs(A[cid(i, j, k + 1)] - A[cid(i, j, k - 1)]) / a / two_dx;
+    // a lane's neighbours lie a plane apart in the interior, a row apart in a
+    // ghost plane: the place of plane 1 and a stride each
+    const double *xm = A + cid(i - 1, j, 1), *xp = A + cid(i + 1, j, 1), *ym = A + cid(i, j - 1, 1),
+                 *yp = A + cid(i, j + 1, 1), *z = A + cid(i, j, 1);
+    const int sxm = i == 1 ? NC : NC * NC, sxp = i == NC ? NC : NC * NC, sym = j == 1 ? NC : NC * NC,
+              syp = j == NC ? NC : NC * NC;
+    double below = A[cid(i, j, 0)], here = *z;
+#pragma unroll 4
+    for (int k = 0; k < NC; k++) {
+      const double above = k == NC - 1 ? A[cid(i, j, NC + 1)] : z[(k + 1) * NC * NC];
+      const double gx = fabs(xp[k * sxp] - xm[k * sxm]) / here / two_dx;
+      const double gy = fabs(yp[k * syp] - ym[k * sym]) / here / two_dx;
+      const double gz = fabs(above - below) / here / two_dx;
       m = fmax(m, fmax(gx, fmax(gy, gz)));
+      below = here;
+      here = above;
     }
   }
   for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
@@ -899,7 +912,8 @@ void plain_finish(const DevCfg &c, const double *UP, double *U, double *P, StepS
 #undef WX_CALL
 }
 static void launch_timestep(const DevCfg &c, const double *P, unsigned long long *slots, hipStream_t st) {
-#define WX_CALL(NV, NF) hipLaunchKernelGGL(k_timestep<NV>, dim3(c.nblk), dim3(256), 0, st, c, P, slots)
+  const int L = planes_for(c.nblk, WX_TIMESTEP_WANT);
+#define WX_CALL(NV, NF) hipLaunchKernelGGL(k_timestep<NV>, dim3(NC / L * c.nblk), dim3(256), 0, st, c, P, slots, L)
   WX_BY_NV(c.nv, WX_CALL);
 #undef WX_CALL
 }
