@@ -71,13 +71,17 @@ def test_download_into_pinned_memory():
     """Memory that the caller pinned takes the state directly (no chunks), at a
     size that ordinary memory takes in chunks; also from its middle on."""
     import ctypes as C
-    import torch
     w, U = _state((13, 7, 1), 6)
     s = hip.Walicxe3D(w, form=hip.FUSED_FP32)
     s.upload(U)
+    L = hip.load()
+    base = C.c_void_p()
+    assert L.hipHostMalloc(C.byref(base), C.c_size_t(U.nbytes + 24), C.c_uint(0)) == 0   # of the runtime it links
+    pin = np.ctypeslib.as_array(C.cast(base, hip._dp), (U.size + 3,))
     for off in (0, 3):
-        pin = torch.zeros(U.size + off, dtype=torch.float64, pin_memory=True)
-        at = C.cast(pin.data_ptr() + 8 * off, hip._dp)
-        assert hip.load().wx_download_state(s._h, at, None, hip.LAYOUT_BLOCKS, 0, None) == 0
-        assert np.array_equal(pin.numpy()[off:].reshape(U.shape), U) and not pin[:off].any()
+        pin[:] = 0.0
+        at = C.cast(base.value + 8 * off, hip._dp)
+        assert L.wx_download_state(s._h, at, None, hip.LAYOUT_BLOCKS, 0, None) == 0
+        assert np.array_equal(pin[off:off + U.size].reshape(U.shape), U) and not pin[:off].any()
     s.close()
+    assert L.hipHostFree(base) == 0

@@ -13,9 +13,16 @@ namespace wx {
 // step: 1053, 1008, 963, 978 us for 512, 1024, 2048, 4096; 512 hydro blocks:
 // 610, 538, 533, 534 us; 64 hydro blocks: 85, 81, 82, 82 us.
 constexpr int WX_UPDATE_WANT = 2048;
-// The same for the timestep pass (one column of 16 planes per lane is a serial
-// chain on a mesh of few blocks).
+// The same for the timestep pass: one column of 16 planes per lane is a serial
+// chain on a mesh of few blocks (getTimestep of 1 MHD block 39 us, in slabs 29).
+// 256, 512, 1024, 2048: 64 MHD blocks 31.9, 31.0, 30.7, 30.6 us, 240: 42.8, 42.4,
+// 41.9, 42.1, 1000: 75.4, 75.9, 72.6, 72.5.
 constexpr int WX_TIMESTEP_WANT = 512;
+// And for the end of the step.  Whole step for 512, 1024, 2048, 4096: 64 viscous
+// hydro blocks 78.0, 82.6, 81.1, 81.5 us, 240: 215, 219, 225, 223, 904: 798, 797,
+// 797, 805; viscous HLLD, 64: 154.6, 157.3, 157.1, 156.6, 240: 485, 479, 474, 477,
+// 904: 1765, 1698, 1665, 1675, 1728: 3177, 3181, 3129, 3101.
+constexpr int WX_FINISH_WANT = 2048;
 
 // ---------------------------------------------------------------------------
 // The device physics routines applied to arrays of records (one thread per
@@ -686,38 +693,46 @@ __global__ void __launch_bounds__(64) k_dt_fold(unsigned long long *slots, unsig
 // the reference.  The reference returns at the first cell whose gradient
 // reaches the refinement threshold; which flag it returns then depends only
 // on the level, so the flag is a function of this maximum (set on the host).
-// grid nblk, block 256: lane (i, j) walks k.
+// One variable at a time is staged in LDS as an 18^3 cube (its edges and
+// corners are not read), every line of the block's interior and inner ghost
+// planes loaded once; the division by the common 2 dx > 0, which keeps the
+// order of the quotients, comes after the maximum.  grid nblk, block 1024.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_mark(DevCfg c, const double *P, double *maxgrad) {
-  __shared__ double part[4];
-  const int b = blockIdx.x;
-  const int i = (threadIdx.x & (NC - 1)) + 1, j = threadIdx.x / NC + 1;
+__global__ void __launch_bounds__(1024) k_mark(DevCfg c, const double *P, double *maxgrad) {
+  constexpr int E = NC + 2;
+  __shared__ double cube[E * E * E];
+  __shared__ double part[16];
+  const int b = blockIdx.x, t = threadIdx.x;
   const double two_dx = 2.0 * c.dx[0][c.info[b].level - 1];
   double m = 0.0;
   for (int s = 0; s < 2; s++) {
     const double *A = P + ((size_t)b * c.nv + (s == 0 ? 4 : 0)) * NSTORE;
-    // a lane's neighbours lie a plane apart in the interior, a row apart in a
-    // ghost plane: the place of plane 1 and a stride each
-    const double *xm = A + cid(i - 1, j, 1), *xp = A + cid(i + 1, j, 1), *ym = A + cid(i, j - 1, 1),
-                 *yp = A + cid(i, j + 1, 1), *z = A + cid(i, j, 1);
-    const int sxm = i == 1 ? NC : NC * NC, sxp = i == NC ? NC : NC * NC, sym = j == 1 ? NC : NC * NC,
-              syp = j == NC ? NC : NC * NC;
-    double below = A[cid(i, j, 0)], here = *z;
-#pragma unroll 4
-    for (int k = 0; k < NC; k++) {
-      const double above = k == NC - 1 ? A[cid(i, j, NC + 1)] : z[(k + 1) * NC * NC];
-      const double gx = fabs(xp[k * sxp] - xm[k * sxm]) / here / two_dx;
-      const double gy = fabs(yp[k * syp] - ym[k * sym]) / here / two_dx;
-      const double gz = fabs(above - below) / here / two_dx;
+    if (s) __syncthreads();
+    for (int q = t; q < NINT; q += 1024)
+      cube[((q / (NC * NC) + 1) * E + (q / NC) % NC + 1) * E + q % NC + 1] = A[q];
+    for (int r = t; r < 6 * 256; r += 1024) {
+      const int f = r >> 8, a1 = (r & 255) % NC + 1, a2 = (r & 255) / NC + 1, gn = (f & 1) ? NC + 1 : 0;
+      const int i = f < 2 ? gn : a1, j = f < 2 ? a1 : (f < 4 ? gn : a2), k = f < 4 ? a2 : gn;
+      cube[(k * E + j) * E + i] = A[cid(i, j, k)];
+    }
+    __syncthreads();
+    for (int q = t; q < NINT; q += 1024) {
+      const int o = ((q / (NC * NC) + 1) * E + (q / NC) % NC + 1) * E + q % NC + 1;
+      const double a = cube[o];
+      const double gx = fabs(cube[o + 1] - cube[o - 1]) / a;
+      const double gy = fabs(cube[o + E] - cube[o - E]) / a;
+      const double gz = fabs(cube[o + E * E] - cube[o - E * E]) / a;
       m = fmax(m, fmax(gx, fmax(gy, gz)));
-      below = here;
-      here = above;
     }
   }
   for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
-  if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = m;
+  if ((t & 63) == 0) part[t >> 6] = m;
   __syncthreads();
-  if (threadIdx.x == 0) maxgrad[b] = fmax(fmax(part[0], part[1]), fmax(part[2], part[3]));
+  if (t == 0) {
+    double r = part[0];
+    for (int w = 1; w < 16; w++) r = fmax(r, part[w]);
+    maxgrad[b] = r / two_dx;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -905,7 +920,7 @@ void plain_viscous(const DevCfg &c, const double *UP, double *U, hipStream_t st)
 }
 void plain_finish(const DevCfg &c, const double *UP, double *U, double *P, StepState *ss, double mu0,
                   unsigned long long *slots, hipStream_t st) {
-  const int L = planes_for(c.nblk, 2048);
+  const int L = planes_for(c.nblk, WX_FINISH_WANT);
 #define WX_CALL(NV, NF)                                                                                          \
   hipLaunchKernelGGL((k_finish<NV, NF>), dim3((NC / L + 12) * c.nblk), dim3(256), 0, st, c, UP, U, P, ss, mu0, slots, L)
   WX_BY_NV(c.nv, WX_CALL);
@@ -930,7 +945,7 @@ void plain_cooling(const DevCfg &c, double *U, double *P, double dt, double mu0,
   hipLaunchKernelGGL(k_cooling, dim3(16, c.nblk), dim3(256), 0, st, c, U, P, dt, mu0);
 }
 void plain_mark(const DevCfg &c, const double *P, double *maxgrad, hipStream_t st) {
-  hipLaunchKernelGGL(k_mark, dim3(c.nblk), dim3(256), 0, st, c, P, maxgrad);
+  hipLaunchKernelGGL(k_mark, dim3(c.nblk), dim3(1024), 0, st, c, P, maxgrad);
 }
 void fused_ghost_prims(const DevCfg &c, const double *U, double *G, hipStream_t st) {
   hipLaunchKernelGGL(k_ghost_prims_fused, dim3(6, c.nblk), dim3(256), 0, st, c, U, G);
