@@ -43,3 +43,20 @@ def test_delta_form_solvers(tmp_path):
     assert r.returncode == 0, r.stderr
     r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
     assert r.returncode == 0 and "delta form ok" in r.stdout, r.stdout + r.stderr
+
+
+@pytest.mark.skipif(not os.path.exists(HIPCC), reason="hipcc not available")
+def test_hllc_select_matches_branches(tmp_path):
+    """The HLLC that every hydro kernel takes (primfhllc_sel) against
+    primfhllc, the form that the reference's vectors check, over all of its
+    outcomes, and the limiters of all variables at once against one by one."""
+    exe = str(tmp_path / "hllc_select")
+    cmd = [HIPCC, "-x", "hip", "-O2", "-ffp-contract=off", "--offload-arch=gfx950",
+           "-I" + os.path.join(ROOT, "walicxe3d_amd", "csrc"), "-I" + os.path.join(ROOT, "include"),
+           os.path.join(HERE, "host", "hllc_select.cpp"), "-o", exe]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr
+    r = subprocess.run([exe], capture_output=True, text=True, timeout=300)
+    assert r.returncode == 0 and "double mismatches 0, float mismatches 0" in r.stdout, r.stdout + r.stderr
+    for reg in ("left", "right", "L*", "R*", "none"):
+        assert ("%s 0 " % reg) not in r.stdout, r.stdout
