@@ -35,7 +35,7 @@ template <typename RF> __device__ __forceinline__ const Phys<RF> &phys(const Dev
 template <> __device__ __forceinline__ const Phys<float> &phys<float>(const DevCfg &c) { return c.pf; }
 template <> __device__ __forceinline__ const Phys<double> &phys<double>(const DevCfg &c) { return c.pd; }
 
-// Riemann solver chosen at compile time (one solver's code per kernel)
+// MHD Riemann solver chosen at compile time (one solver's code per kernel)
 #ifdef WX_NOINLINE_RIEMANN
 #define WX_RIEMANN_INLINE __noinline__
 #else
@@ -45,16 +45,15 @@ template <> __device__ __forceinline__ const Phys<double> &phys<double>(const De
 // one code path)
 template <int SOLVER, typename RF, bool S1 = false>
 __device__ WX_RIEMANN_INLINE void riemann_t(const Phys<RF> &P, const RF *pl, const RF *pr, RF *ff) {
-  if constexpr (SOLVER == SOLVER_HLLC) primfhllc(P, pl, pr, ff);
-  else if constexpr (SOLVER == SOLVER_HLLD) {
+  static_assert(SOLVER == SOLVER_HLLD || SOLVER == SOLVER_HLLE, "MHD");
+  if constexpr (SOLVER == SOLVER_HLLD) {
 #ifdef WX_HLLD_BRANCHES
     primfhlld(P, pl, pr, ff);
 #else
     primfhlld_sel<RF, S1 && sizeof(RF) == 4>(P, pl, pr, ff);
 #endif
   }
-  else if constexpr (SOLVER == SOLVER_HLLE) primfhlle(P, pl, pr, ff);
-  else primfhll(P, pl, pr, ff);
+  else primfhlle(P, pl, pr, ff);
 }
 
 // a value that is the same in every lane, read from the first active lane
@@ -424,22 +423,23 @@ __device__ __forceinline__ void finish_cell(const FusedArgs &a, int b, int i, in
 }
 
 // ---------------------------------------------------------------------------
-// Stage kernel.  S2 = second stage; VISC = artificial viscosity active;
-// RF = flux/reconstruction arithmetic; ST = storage type of UP; SOLVER =
-// Riemann solver; LIM = limiter fixed at compile time, or LIM_RUNTIME.
-// Launch bound: 256 threads, at least three waves per SIMD (four for the MHD
-// first stage).
+// Stage kernel of MHD with plain FP32 fluxes.  S2 = second stage; VISC =
+// artificial viscosity active; SOLVER = Riemann solver; LIM = limiter fixed at
+// compile time, or LIM_RUNTIME.  Launch bound: 256 threads, at least three
+// waves per SIMD (four for the first stage).
 // ---------------------------------------------------------------------------
 #ifndef WX_STAGE_MIN_WAVES
 #define WX_STAGE_MIN_WAVES 3
 #endif
-// the MHD first stage (no limiter, fewer live values) runs best at four
+// the first stage (no limiter, fewer live values) runs best at four
 #ifndef WX_MHD_STAGE1_MIN_WAVES
 #define WX_MHD_STAGE1_MIN_WAVES 4
 #endif
-template <int NV, bool S2, bool VISC, typename RF, typename ST, int SOLVER, int LIM>
-__global__ void __launch_bounds__(256, (NV == 8 && !S2) ? WX_MHD_STAGE1_MIN_WAVES : WX_STAGE_MIN_WAVES)
-    k_stage(FusedArgs a) {
+template <bool S2, bool VISC, int SOLVER, int LIM>
+__global__ void __launch_bounds__(256, S2 ? WX_STAGE_MIN_WAVES : WX_MHD_STAGE1_MIN_WAVES) k_stage(FusedArgs a) {
+  constexpr int NV = 8;
+  using RF = float;   // flux and reconstruction arithmetic
+  using ST = float;   // storage of UP
   constexpr int ORD = S2 ? 2 : 1;
   constexpr int H = ORD;
   constexpr int W = NC + 2 * H;
@@ -703,30 +703,26 @@ __global__ void __launch_bounds__(256, (NV == 8 && !S2) ? WX_MHD_STAGE1_MIN_WAVE
   }
 }
 
-// second-stage kernels with the limiter fixed at compile time (minmod, in
-// the FP32 MHD form) or read at run time
-template <typename RF, typename ST, int NV, int SOLVER, bool VISC>
+// second-stage kernels with the limiter fixed at compile time (minmod) or read
+// at run time
+template <int SOLVER, bool VISC>
 inline void launch_stage2(const FusedArgs &a, int grid, hipStream_t st) {
   constexpr int MM = 1;  // LIMITER_MINMOD (source/constants.f90)
-  if constexpr (sizeof(RF) == 4 && NV == 8) {
-    if (a.c.pf.limiter == MM) {
-      hipLaunchKernelGGL((k_stage<NV, true, VISC, RF, ST, SOLVER, MM>), dim3(grid), dim3(256), 0, st, a);
-      return;
-    }
-  }
-  hipLaunchKernelGGL((k_stage<NV, true, VISC, RF, ST, SOLVER, LIM_RUNTIME>), dim3(grid), dim3(256), 0, st, a);
+  if (a.c.pf.limiter == MM)
+    hipLaunchKernelGGL((k_stage<true, VISC, SOLVER, MM>), dim3(grid), dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL((k_stage<true, VISC, SOLVER, LIM_RUNTIME>), dim3(grid), dim3(256), 0, st, a);
 }
 
-template <typename RF, typename ST, int NV, int SOLVER>
+template <int SOLVER>
 inline void launch_stage_s(const FusedArgs &a, int grid, bool visc, int stage, hipStream_t st) {
   if (stage == 1)
-    hipLaunchKernelGGL((k_stage<NV, false, false, RF, ST, SOLVER, LIM_RUNTIME>), dim3(grid), dim3(256), 0, st, a);
+    hipLaunchKernelGGL((k_stage<false, false, SOLVER, LIM_RUNTIME>), dim3(grid), dim3(256), 0, st, a);
   else if (visc)
-    launch_stage2<RF, ST, NV, SOLVER, true>(a, grid, st);
+    launch_stage2<SOLVER, true>(a, grid, st);
   else
-    launch_stage2<RF, ST, NV, SOLVER, false>(a, grid, st);
+    launch_stage2<SOLVER, false>(a, grid, st);
 }
-
 
 // FP32 MHD stage kernels (HLLD, HLLE), defined in wx_fused_mhd.hip: the
 // delta-form kernels, or with plain32 the plain FP32 flux kernels above

@@ -14,8 +14,8 @@ namespace wx {
 
 void launch_stage_mhd32(const FusedArgs &a, int grid, int solver, bool visc, int stage, int plain32, hipStream_t st) {
   if (plain32) {
-    if (solver == SOLVER_HLLD) launch_stage_s<float, float, 8, SOLVER_HLLD>(a, grid, visc, stage, st);
-    else launch_stage_s<float, float, 8, SOLVER_HLLE>(a, grid, visc, stage, st);
+    if (solver == SOLVER_HLLD) launch_stage_s<SOLVER_HLLD>(a, grid, visc, stage, st);
+    else launch_stage_s<SOLVER_HLLE>(a, grid, visc, stage, st);
     return;
   }
   if (solver == SOLVER_HLLD) launch_mhd<SOLVER_HLLD>(a, grid, stage, st);
