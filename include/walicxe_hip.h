@@ -70,7 +70,9 @@ typedef struct wx_config {
   const double *tab_loglam;  /* log10(Lambda) */
   int nwind;                 /* spherical wind sources re-imposed at every */
   const double *winds;       /* boundary call (winds.f90:123): 8 per source:
-                                xc,yc,zc,radius,mdot,vinf,temp,mu (cgs)   */
+                                xc,yc,zc,radius,mdot,vinf,temp,mu (cgs);
+                                MHD with sources: the plain FP64 and the
+                                fused FP32 form (else WX_EINVAL)          */
   int form;                  /* WX_FORM_* */
 } wx_config;
 

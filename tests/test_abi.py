@@ -136,3 +136,28 @@ def test_noalloc_eval_refuses_more_than_its_staging():
     assert rc == -1
     assert b"staging" in L.wx_last_error()
     assert L.wx_eval_physics_noalloc(C.byref(cfg), 99, 0, 1, a.ctypes.data_as(dp), out.ctypes.data_as(dp)) == -1
+
+
+def test_fused_fp64_mhd_with_wind_sources_is_refused():
+    """The combination that no GPU test has run is refused before a device is
+    touched; hydro with sources and MHD without pass these checks (and fail,
+    without a GPU, at the device query only)."""
+    if not os.path.exists(hip.LIBPATH):
+        pytest.skip("library not built")
+    import dataclasses
+    from walicxe3d_amd import workloads as W
+    L = hip.load()
+    h = C.c_void_p()
+    for solver in ("hlld", "hlle"):
+        cfg = hip.make_config(dataclasses.replace(W.get("mhd_winds4"), solver=solver), form=hip.FUSED_FP64)
+        assert cfg.nwind == 3
+        assert L.wx_init(C.byref(cfg), C.byref(h)) == -1
+        assert b"MHD with wind sources" in L.wx_last_error()
+    for name, form in (("winds4", hip.FUSED_FP64), ("ot64", hip.FUSED_FP64), ("mhd_winds4", hip.PLAIN_FP64),
+                       ("mhd_winds4", hip.FUSED_FP32)):
+        cfg = hip.make_config(W.get(name), form=form)
+        rc = L.wx_init(C.byref(cfg), C.byref(h))
+        if rc == 0:
+            L.wx_finalize(h)
+        else:
+            assert rc != -1, L.wx_last_error()

@@ -1025,6 +1025,10 @@ int wx_init(const wx_config *cfg, void **out) {
     return fail(WX_EINVAL, "the fused form with nv = 8 runs HLLE or HLLD");
   if (cfg->form != WX_FORM_PLAIN_FP64 && cfg->nv == 8 && !cfg->mhd)
     return fail(WX_EINVAL, "the fused form with nv = 8 needs mhd = 1");
+  // no GPU run has ever completed in this combination: one that held it among
+  // other wind cases ended in a GPU fault whose cause is not known
+  if (cfg->form == WX_FORM_FUSED_FP64 && cfg->nv == 8 && cfg->nwind)
+    return fail(WX_EINVAL, "MHD with wind sources runs in the plain FP64 and the fused FP32 form");
   // calcTemp (source/hydro_core.f90:231-270): EOS_H_RATE (3) takes the
   // neutral hydrogen density from the first passive scalar (plain form)
   if (cfg->eos < 0 || cfg->eos > 3)

@@ -298,19 +298,26 @@ static void launch_flow_t(const FusedArgs &a, int grid, int stage, hipStream_t s
 
 template <int NV, typename RF, typename ST, int SOLVER>
 static void launch_flow(const FusedArgs &a, int grid, int stage, hipStream_t st) {
-  if (a.c.nwind > 0) launch_flow_t<NV, RF, ST, SOLVER, true>(a, grid, stage, st);
-  else launch_flow_t<NV, RF, ST, SOLVER, false>(a, grid, stage, st);
+  if constexpr (NV == 5) {   // FP64 MHD has no wind sources (wx_init)
+    if (a.c.nwind > 0) return launch_flow_t<NV, RF, ST, SOLVER, true>(a, grid, stage, st);
+  }
+  launch_flow_t<NV, RF, ST, SOLVER, false>(a, grid, stage, st);
 }
 
 template <int NV, typename RF, typename ST>
 static void launch_end(const FusedArgs &a, hipStream_t st) {
   const int grid = a.nblk * a.nslab;
-  if (a.c.visc_eta == 0.0)
+  if (a.c.visc_eta == 0.0) {
     hipLaunchKernelGGL((k_end<NV, RF, ST, false, false, false>), dim3(grid), dim3(256), 0, st, a);
-  else if (a.c.nwind > 0)
-    hipLaunchKernelGGL((k_end<NV, RF, ST, true, false, true>), dim3(grid), dim3(256), 0, st, a);
-  else
-    hipLaunchKernelGGL((k_end<NV, RF, ST, true, false, false>), dim3(grid), dim3(256), 0, st, a);
+    return;
+  }
+  if constexpr (NV == 5) {
+    if (a.c.nwind > 0) {
+      hipLaunchKernelGGL((k_end<NV, RF, ST, true, false, true>), dim3(grid), dim3(256), 0, st, a);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_end<NV, RF, ST, true, false, false>), dim3(grid), dim3(256), 0, st, a);
 }
 
 // slabs per block that give `want` workgroups, at least `least`
