@@ -28,8 +28,8 @@ Summary mode:
         --workload ot256 --out profiles/stage2_ot256_traffic.txt [--cmd "..."]
 reads the two counter_collection.csv files (FETCH_SIZE and WRITE_SIZE, KiB
 per dispatch), takes the copy kernel's readings as the scale (bytes moved /
-counter), and writes per-launch HBM traffic of the stage kernels next to
-their algorithmic bytes.
+counter), and writes per-launch HBM traffic of the stage kernels, and of the
+kernel that ends a step where there is one, next to their algorithmic bytes.
 
 Counter table mode:
     python3 -m walicxe3d_amd.profile_run counters --dirs DIR [DIR ...] \
@@ -177,7 +177,8 @@ def _summarize(args):
     write = _per_kernel(_read(args.write), "WRITE_SIZE")
     fscale = COPY_BYTES / (1024.0 * _copy_reading(fetch))
     wscale = COPY_BYTES / (1024.0 * _copy_reading(write))
-    alg = {"stage1": zones * w.nv * (8 + 4), "stage2": zones * w.nv * (4 + 8 + 8)}
+    # end: the state that the second stage left, in and out
+    alg = {"stage1": zones * w.nv * (8 + 4), "stage2": zones * w.nv * (4 + 8 + 8), "end": zones * w.nv * (8 + 8)}
     lines = ["# HBM traffic of the fused stage kernels, %s (%d blocks, %d zones, nv=%d)" %
              (w.name, len(w.blocks()), zones, w.nv),
              "# command: %s" % (args.cmd or "(see walicxe3d_amd/profile_run.py)"),
@@ -196,7 +197,7 @@ def _summarize(args):
         wr = sum(v for _, _, v in write.get(k, [(0, 0, 0.0)])) / max(1, len(write.get(k, [])))
         hbm = 1024.0 * (f * fscale + wr * wscale)
         out[st] = (k, f, wr, hbm)
-    for st in ("stage1", "stage2"):
+    for st in ("stage1", "stage2", "end"):
         if st not in out:
             continue
         k, f, wr, hbm = out[st]
@@ -206,7 +207,10 @@ def _summarize(args):
                   "%s_hbm_bytes_per_launch = %.4e" % (st, hbm),
                   "%s_algorithmic_bytes_per_launch = %.4e" % (st, alg[st]),
                   "%s_traffic_over_algorithmic = %.3f" % (st, hbm / alg[st])]
-    if "stage2" in out:
+    if "end" in out:
+        lines += ["", "hbm_bytes_per_launch = %.4e   (stage 2 with the end of the step)"
+                  % (out["stage2"][3] + out["end"][3])]
+    elif "stage2" in out:
         lines += ["", "hbm_bytes_per_launch = %.4e   (stage 2, the dominant kernel)" % out["stage2"][3]]
     text = "\n".join(lines) + "\n"
     if args.out:
@@ -226,7 +230,10 @@ def _header(args, title):
 
 
 def _stage_of(k):
-    """'stage1' / 'stage2' for a fused stage kernel name, else None."""
+    """'stage1' / 'stage2' for a fused stage kernel name, 'end' for the kernel
+    that ends a step, else None."""
+    if "k_end<" in k:
+        return "end"
     if not any(n in k for n in ("k_stage<", "k_flow<", "k_mhd<")):
         return None
     targs = k.split("<", 1)[1].split(",")
