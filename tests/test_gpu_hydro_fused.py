@@ -4,8 +4,9 @@ end of the step in its own kernel), so without viscosity every state is the
 same bit for bit.  The viscous sum takes the two z neighbours in the other
 order (the column is walked upwards): 2 ulp of a term weighted by 5e-3, so a
 cell's last bit changes now and then; 1e-13 of a variable's largest value is
-over a hundred such flips per step.  The FP32 form is the same code in another type; its error is bounded in
-test_gpu_parity.py."""
+over a hundred such flips per step.  The FP32 kernels are the same templates,
+but only they keep their halo's sources in tables, checked at the end of this
+file; their error is bounded in test_gpu_parity.py."""
 import dataclasses
 
 import numpy as np
@@ -54,8 +55,9 @@ def test_fused_fp64_hydro_equals_the_plain_form(name, visc, limiter):
     assert _same(a, b, visc == 0.0)
 
 
-# 1 to 1024 blocks, and counts that are no multiple of 8: every slab count of
-# the stages (16 to 1) and of the end of the step, and the tail of the dealing
+# 1 to 1024 blocks, and counts that are no multiple of 8: slab counts 16 to 2 of
+# the stages (whole blocks: test_whole_blocks) and every one of the end of the
+# step, and the tail of the dealing
 @pytest.mark.parametrize("nroot", [(1, 1, 1), (3, 1, 1), (8, 2, 1), (5, 5, 1), (16, 3, 1), (16, 4, 1), (16, 8, 1)])
 @pytest.mark.parametrize("base,visc", [(1, 0.0), (2, 0.0), (1, 5.0e-3), (2, 5.0e-3)])
 def test_slab_counts(nroot, base, visc):

@@ -15,10 +15,11 @@
 // dt candidate) in FP64 on U^{n+1}; dt reduced as an exact min.
 //
 // Stage 1 (first order, dt/2): U^n (FP64) -> UP (FP32).
-// Stage 2 (second order, dt): UP, U^n -> U^{n+1}, with the next dt.  With
-// artificial viscosity or cooling stage 2 leaves its state to k_end, which
-// applies both (the viscosity's face neighbours are the half-step ghosts, as
-// in the reference) and forms the next dt.
+// Stage 2 (second order, dt): UP, U^n -> U^{n+1}.  Hydro and FP64 leave that
+// state to k_end, which applies viscosity (its face neighbours are the
+// half-step ghosts, as in the reference) and cooling and forms the next dt;
+// FP32 MHD does so with viscosity or cooling only, else its stage 2 ends the
+// step itself.
 // k_flow (hydro, FP64 MHD; wx_hydro_kern.h), k_mhd (FP32 MHD;
 // wx_mhd_kern.h), k_stage (MHD with plain FP32 fluxes, set_tuning kind 3).
 #include <hip/hip_runtime.h>
@@ -43,6 +44,12 @@ namespace wx {
 // 51.0, 50.5, 52.6 for 256, 512, 1024.  FP32 MHD (two workgroups per CU) takes
 // slabs below MHD_WANT unless set_tuning chose: 64 blocks 83.4, 65.7, 76.3 for
 // 256, 512, 1024; 32 blocks 56.2, 47.3, 46.9; whole blocks took 265 and 270.
+// FP64 (hydro and MHD, two to three workgroups per CU) shares HYDRO_WANT, whole
+// step for 512, 1024, 2048, 4096: HLLC without viscosity, 64 blocks 64.0, 70.6, 70.8,
+// 71.1 us, 240 153, 163, 188, 185, 904 497, 478, 479, 508, 1728 871, 871, 863, 894;
+// HLLD, 64 116, 133, 136, 131, 240 338, 350, 387, 384, 904 1199, 1174, 1151, 1213, 1728
+// 2078, 2077, 2059, 2103: 2048 is the better line from 904 blocks on, and 10 to 19
+// per cent behind 512 (planes enough to pay for a slab's extra ones) at 64 and 240.
 constexpr int HYDRO_WANT = 2048, END_WANT = 512, MHD_WANT = 512;
 
 static thread_local std::string f_err;

@@ -8,15 +8,19 @@
 // own: it needs the updated neighbours of a cell, which inside the second
 // stage means carrying two more planes of FP64 state, and the cooling's
 // transcendentals, through the flux code, at a third of the registers spilled
-// (162 VGPRs for HLLC); apart, both run without spills, thin slabs need no
-// recomputed planes, and the state in between costs 16 B per variable and
-// zone.
+// (162 VGPRs for HLLC).  Apart, the FP32 stages hold all their values (with wind
+// sources and a run-time limiter 2 to 3 VGPRs go to scratch), and the end of the
+// step all but 36 bytes a lane of a few instances; the FP64 MHD second stage
+// still puts out 9 VGPRs (HLLE with minmod) to 25 (a run-time limiter).  Thin
+// slabs need no recomputed planes.  The state in between costs 16 B per variable
+// and zone, also where there is neither viscosity nor cooling (25 of 375 us for
+// 240 FP64 MHD blocks).
 //
-// Bound: VALU issue at 4 waves per SIMD (stages, 128 VGPRs) and 3 (end of the
-// step).  1728 blocks, HLLC with viscosity: first stage 450 -> 208 us, second
-// 878 -> 278 + 273 us (end); 904 blocks on 4 levels with cooling 299 -> 134 and
-// 784 -> 167 + 210 us; 64 blocks, where one workgroup per block left 192 of 256
-// CUs idle, 127 -> 14 and 221 -> 17 + 15 us.
+// Bound: VALU issue at 4 waves per SIMD (FP32 stages, 128 VGPRs), memory and its
+// latency at 3 (end of the step).  1728 blocks, HLLC with viscosity: first stage
+// 450 -> 187 us, second 878 -> 238 + 210 us (end); 904 blocks on 4 levels with
+// cooling 299 -> 121 and 784 -> 157 + 184 us; 64 blocks, where one workgroup per
+// block left 192 of 256 CUs idle, 127 -> 14 and 221 -> 16 + 10 us.
 #pragma once
 
 #include <type_traits>

@@ -19,8 +19,10 @@
 // reads U^n of neighbour blocks for its halo and so writes U^{n+1} into the
 // second state buffer (the two swap roles every step).
 //
-// Bound: VALU issue and latency at the 2 waves per SIMD that 256 VGPRs and
-// 67 KB of LDS leave.  The x/y halo used to ask for its source cell in every
+// Bound: memory and VALU issue alike, at the 2 waves per SIMD that 256 VGPRs
+// and 67 KB of LDS leave: of the 1.29 ms of the second stage on 4096 HLLD blocks
+// 0.89 are VALU issue, and its 5.3 GB read and 1.1 written are 5.0 TB/s (reads
+// alone reach 5.9 on this card, a copy 4.75).  The x/y halo used to ask for its source cell in every
 // plane, between two barriers; now the sources are found once per block
 // (HaloRef, ColRef), the loads of the next plane are issued before the last
 // barrier of this one, two barriers a plane remain of three, the waves take
@@ -29,7 +31,7 @@
 // With viscosity or cooling the second stage leaves its state to k_end (TO_X):
 // inside, that code held one workgroup per CU (82 KB of LDS) and spilled.
 // 8 viscous HLLE blocks, whole blocks -> 16 slabs: first stage 81 -> 10 us,
-// second 275 -> 23 + 9 us.
+// second 275 -> 22 + 7 us.
 #pragma once
 
 #include "wx_delta.h"
@@ -529,14 +531,21 @@ __global__ void __launch_bounds__(256, WX_MHD_MIN_WAVES) k_mhd(FusedArgs a) {
   }
 }
 
-// with viscosity or cooling the second stage leaves its state to k_end (to_x)
+// With viscosity or cooling the second stage leaves its state to k_end (to_x):
+// one instance, with the wind code and the limiter read at run time, also for
+// meshes without sources and for minmod.  Contraction fuses some sums of xflux
+// from one side or the other as the code around them changes, and an instance
+// without that code rounded them the other way; this one keeps the results that
+// the kernel with viscosity inside gave.  It spills 13 VGPRs (HLLD; HLLE 5) and
+// loads no plane ahead: 1728 viscous HLLD blocks 2.03 ms a step with k_end (1.43
+// without viscosity; 3.04 with the viscosity inside), 64 blocks 105 us (451).
 template <int SOLVER, bool WIND>
 inline void launch_mhd_w(const FusedArgs &a, int grid, bool to_x, int stage, hipStream_t st) {
   constexpr int MM = 1;  // LIMITER_MINMOD (source/constants.f90)
   const bool mm = a.c.pf.limiter == MM && !WIND;
   if (stage == 1)
     hipLaunchKernelGGL((k_mhd<false, false, SOLVER, LIM_RUNTIME, WIND>), dim3(grid), dim3(256), 0, st, a);
-  else if (to_x)   // one instance for meshes with and without sources
+  else if (to_x)
     hipLaunchKernelGGL((k_mhd<true, true, SOLVER, LIM_RUNTIME, true>), dim3(grid), dim3(256), 0, st, a);
   else if (mm)
     hipLaunchKernelGGL((k_mhd<true, false, SOLVER, MM, false>), dim3(grid), dim3(256), 0, st, a);
