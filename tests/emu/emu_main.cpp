@@ -126,7 +126,8 @@ static int run_case(const char *path, int nsteps) {
     std::vector<double> P(U.size());
     if (counted("get_timestep", [&] { return wx_get_timestep(ctx, &raw); }) < 0) return 1;
     if (counted("download", [&] { return wx_download_state(ctx, U.data(), P.data(), WX_LAYOUT_BLOCKS, 0, nullptr); }) < 0) return 1;
-    if (counted("plain_host", [&] { return wx_download_state(ctx, U.data(), nullptr, WX_LAYOUT_BLOCKS, 0, nullptr); }) < 0) return 1;
+    for (int n = 0; n < 8; n++)
+      if (counted(("plain_host" + std::to_string(n)).c_str(), [&] { return wx_download_state(ctx, U.data(), nullptr, WX_LAYOUT_BLOCKS, 0, nullptr); }) < 0) return 1;
     emu_pinned = P.data();
     emu_pinned_bytes = 8 * P.size();
     if (counted("pinned_host", [&] { return wx_download_state(ctx, P.data(), nullptr, WX_LAYOUT_BLOCKS, 0, nullptr); }) < 0) return 1;

@@ -214,35 +214,19 @@ def test_no_call_holds_a_state_more_than_an_upload(emu, tmp_path, name, form, he
         assert c[call]["peak"] <= lim, (call, c[call]["peak"] / one)
 
 
-def test_pinned_destinations_are_copied_to_directly(emu, tmp_path):
-    """A download of 10 MB goes through the lanes' chunks to ordinary memory
-    and in one copy to memory that the caller pinned."""
+def test_destinations_of_downloads(emu, tmp_path):
+    """Downloads of 10 MB to ordinary memory go in one copy each until the
+    pinned chunks pay (40 MB have gone by), then through chunks of 1 MB; to
+    memory that the caller pinned always in one copy."""
     w = W.get("sedov")
     c, U0 = _counts(emu, tmp_path, "pinned", w, hip.FUSED_FP32)
     assert U0.nbytes > (8 << 20)
-    assert c["plain_host"]["copies"] == -(-U0.nbytes // (1 << 20))
+    # the case itself has made some downloads before
+    copies = [c["plain_host%d" % n]["copies"] for n in range(8)]
+    chunks = -(-U0.nbytes // (1 << 20))
+    assert set(copies) <= {1, chunks} and copies == sorted(copies) and copies[4:] == [chunks] * 4
+    assert c["download"]["copies"] < 2 * chunks
     assert c["pinned_host"]["copies"] == 1
-
-
-@pytest.mark.parametrize("name", ["amr_small", "blast_reflect", "ot64_amr", "mhd_hlle"])
-def test_halo_tables_equal_the_general_lookup(emu, tmp_path, monkeypatch, name):
-    """Where a block's halo cells lie, found once per block (halo_ref; in MHD
-    also col_ref), against ghost_source asked for every cell: a wind source of
-    radius 0 covers nothing and picks the instances without tables (in MHD the
-    x/y table stays).  Open, reflective, periodic, coarser, finer and
-    same-level faces; the states are the same bit for bit."""
-    import dataclasses
-    w = W.get(name)
-    boxes = [w.bc] if name != "ot64_amr" else [w.bc, ("reflective", "free", "free", "reflective", "reflective", "free")]
-    for n, bc in enumerate(boxes):
-        outs = []
-        for winds in ([], [(0.0, 0.0, 0.0, 0.0, 1.0, 1.0, 1.0e4, 1.0)]):
-            monkeypatch.setattr(W, "wind_params", lambda w, v=winds: v)
-            p = str(tmp_path / ("halo%d_%d.bin" % (n, len(winds))))
-            _write_input(p, dataclasses.replace(w, bc=bc), hip.FUSED_FP32)
-            _run(emu, [p, "1"], str(tmp_path))
-            outs.append(np.fromfile(p + ".out"))
-        assert np.array_equal(outs[0], outs[1]), bc
 
 
 def test_slab_count_of_the_rule_can_be_set_and_given_back(emu, tmp_path):

@@ -493,6 +493,10 @@ int launch_check(const char *what) {
 // 25 ms; 283 MB 27 -> 7, 10 MB 1.2 -> 0.4.  Chunks of 1 MB leave gaps between
 // the copies (35 ms for 1.07 GB, 2 MB 28, 4 MB 25), but their buffers are
 // pinned sooner, so they grow with the transfer; 8 lanes are no faster than 4.
+// Pinning 8 MB takes 0.7 to 1.3 ms, what four downloads of 10 MB save: the
+// first transfers of a process take the runtime's path until HOST_PAYS times
+// the buffers' bytes have gone by (the first one of 4 MB 0.95 -> 0.3 ms, of 10
+// MB 1.6 -> 1.0; from 84 MB on the first one pays).
 // The buffers (8 to 32 MB) belong to the process, one transfer at a time uses
 // them (another one meanwhile takes the runtime's path), and the last context
 // gives them back.
@@ -502,12 +506,22 @@ size_t host_chunk(size_t bytes) {
   return bytes < (size_t(32) << 20) ? size_t(1) << 20 : (bytes < (size_t(256) << 20) ? size_t(2) << 20 : size_t(4) << 20);
 }
 
+constexpr size_t HOST_PAYS = 5;
+
 struct HostLanes {
   std::mutex busy;      // held by the transfer that uses the buffers
+  size_t passed = 0;    // bytes of transfers that found them too small
   std::mutex count;     // guards users
   int users = 0;        // contexts alive
   char *buf = nullptr;
   size_t size = 0;
+  // whether a transfer of `bytes` may have buffers of `need` bytes pinned for
+  // it (the caller holds busy)
+  bool pays(size_t bytes, size_t need) {
+    if (size >= need) return true;
+    passed += bytes;
+    return passed >= HOST_PAYS * need;
+  }
   // buffers of at least `need` bytes (the caller holds busy)
   bool grow(size_t need) {
     if (size >= need) return true;
@@ -532,7 +546,7 @@ struct HostLanes {
     std::lock_guard<std::mutex> b(busy);
     if (buf) hipHostFree(buf);
     buf = nullptr;
-    size = 0;
+    size = passed = 0;
   }
 };
 HostLanes g_lanes;
@@ -581,8 +595,9 @@ int to_host(Ctx *c, double *dst, const double *src, size_t n) {
   const size_t bytes = n * sizeof(double);
   std::unique_lock<std::mutex> use(g_lanes.busy, std::defer_lock);
   if (bytes >= HOST_MIN && pageable(dst) && use.try_lock()) {
-    const size_t chunk = host_chunk(bytes);
-    if (g_lanes.grow(2 * HOST_LANES * chunk)) {
+    size_t chunk = host_chunk(bytes);
+    if (!g_lanes.pays(bytes, 2 * HOST_LANES * chunk)) chunk = g_lanes.size / (2 * HOST_LANES);   // those there are, if any
+    if (chunk && g_lanes.grow(2 * HOST_LANES * chunk)) {
       hipError_t err[HOST_LANES];
       std::thread th[HOST_LANES];
       char *d = reinterpret_cast<char *>(dst);
