@@ -229,6 +229,27 @@ def test_destinations_of_downloads(emu, tmp_path):
     assert c["pinned_host"]["copies"] == 1
 
 
+@pytest.mark.parametrize("name", ["amr_small", "blast_reflect", "ot64_amr", "mhd_hlle"])
+def test_halo_tables_equal_the_general_lookup(emu, tmp_path, monkeypatch, name):
+    """Where a block's halo cells lie, found once per block (halo_ref; in MHD
+    also col_ref), against ghost_source asked for every cell: a wind source of
+    radius 0 covers nothing and picks the instances without tables (in MHD the
+    x/y table stays).  Open, reflective, periodic, coarser, finer and
+    same-level faces; the states are the same bit for bit."""
+    import dataclasses
+    w = W.get(name)
+    boxes = [w.bc] if name != "ot64_amr" else [w.bc, ("reflective", "free", "free", "reflective", "reflective", "free")]
+    for n, bc in enumerate(boxes):
+        outs = []
+        for winds in ([], [(0.0, 0.0, 0.0, 0.0, 1.0, 1.0, 1.0e4, 1.0)]):
+            monkeypatch.setattr(W, "wind_params", lambda w, v=winds: v)
+            p = str(tmp_path / ("halo%d_%d.bin" % (n, len(winds))))
+            _write_input(p, dataclasses.replace(w, bc=bc), hip.FUSED_FP32)
+            _run(emu, [p, "1"], str(tmp_path))
+            outs.append(np.fromfile(p + ".out"))
+        assert np.array_equal(outs[0], outs[1]), bc
+
+
 def test_slab_count_of_the_rule_can_be_set_and_given_back(emu, tmp_path):
     """Kind 4 takes every count the rule by mesh size can choose (16 on these
     8 blocks, viscous and inviscid) and 0 for the rule itself: the same state
